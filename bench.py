@@ -467,8 +467,7 @@ def main() -> int:
     ap.add_argument("--copy-probe", type=int, default=0, metavar="MIB",
                     help="only run the streaming probe kernels on MIB MiB (to calibrate HBM byte counters)")
     ap.add_argument("--tendency-form", choices=("default", "separate", "fused"), default="default",
-                    help="tendencies in a kernel of their own (separate, the default) or formed inside the "
-                         "friction + AB kernel (fused)")
+                    help="ps3d_set_fused_tendency: accepted, both run the same kernels")
     args = ap.parse_args()
     if args.copy_probe:
         # the library's streaming kernels only (k_copy moves 2 x MIB MiB per

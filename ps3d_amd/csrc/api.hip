@@ -284,11 +284,6 @@ void integrate(Model &m, int itt, int tau, int taum1, int taum2)
         return;
     }
     const bool forced = m.forcing || m.wm_on || background_on(m);
-    if (fused_tendency_active(m)) {
-        launch_friction_ab(m, itt, tau, taum1, taum2, true);   // tendency formed inside
-        pressure(m);
-        return;
-    }
     launch_tendency(m, tau);
     if (fused_friction_ok(m) && m.fuse_friction && !forced) {
         launch_friction_ab(m, itt, tau, taum1, taum2);
@@ -363,7 +358,7 @@ std::vector<uint64_t> graph_signature(const Model &m, const int32_t *st)
     uint64_t h = 1469598103934665603ull;
     h = fnv(h, &m.c, sizeof(m.c));
     h = fnv(h, &m.prm, sizeof(m.prm));
-    const int opts[] = {m.tend_kc, m.fric_kc, m.tfric_kc, m.thomas_cpw, (int)m.thomas_reg, (int)m.fuse_tendency,
+    const int opts[] = {m.tend_kc, m.fric_kc, m.thomas_cpw, (int)m.thomas_reg,
                         (int)m.fuse_friction, (int)m.fuse_halo, m.fft_plan[0], m.fft_plan[1], m.fft_plan[2],
                         (int)m.bg_on, (int)m.bg_b_on, (int)m.bf_on[0], (int)m.bf_on[1], (int)m.bf_on[2],
                         (int)m.bf_on[3]};
@@ -412,7 +407,7 @@ void capture_steps(Model &m, const int32_t *st)
 }
 
 const char *kKernelNames =
-    "tendency,friction_ab,tend_friction_ab,harmonic,biharmonic_h,biharmonic_v,ab_update,halo,fft_x_r2c,fft_y_fwd,thomas,"
+    "tendency,friction_ab,harmonic,biharmonic_h,biharmonic_v,ab_update,halo,fft_x_r2c,fft_y_fwd,thomas,"
     "fft_y_inv,fft_x_c2r,z_solve,fft_z_fwd,fft_z_inv,project";
 
 }  // namespace
@@ -1062,7 +1057,6 @@ int ps3d_set_fused_tendency(ps3d_model *m, int on)
     return guard([&] {
         check_model(m);
         PS3D_REQUIRE(on == 0 || on == 1, "on must be 0 or 1");
-        m->fuse_tendency = on != 0;
     });
 }
 

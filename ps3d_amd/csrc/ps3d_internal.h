@@ -217,10 +217,6 @@ struct Model {
     int cur[4] = {0, 0, 0, 0};
     // use the fused friction + Adams-Bashforth kernel where it applies
     bool fuse_friction = true;
-    // form the tendency inside it (unforced FP64 steps): reads the state
-    // once and never reads slot tau back, but measured slower than the
-    // separate tendency kernel (ps3d_set_fused_tendency), so off by default
-    bool fuse_tendency = false;
     // producers write the halo images of what they update (halo_images_ok)
     bool fuse_halo = false;
     // launch shapes (results do not depend on them; set by ps3d_tune):
@@ -230,7 +226,6 @@ struct Model {
     // lanes; 16, 32, 64 columns per wave on the fly; -16, -32, -64 the factor
     // tables; 0: the heuristic)
     int tend_kc = 0, fric_kc = 0, thomas_cpw = 0;
-    int tfric_kc = 0;   // the same for the kernel with the tendency fused in
     // the heuristic's first choice: whole columns in registers where nz is
     // one of the compiled-in column lengths (k_thomas_reg)
     bool thomas_reg = true;
@@ -311,9 +306,7 @@ void launch_background(Model &m, int tau, float *const *mixed_fields = nullptr);
 void launch_friction_forcing_ab_mixed(Model &m, int itt, int tau, int taum1, int taum2, double qc1, const float *d1,
                                       double qc2, const float *d2);
 bool fused_friction_ok(const Model &m);
-// with_tendency: the tendency of integrate.f90:12-54 formed in the same
-// kernel (k_tend_fric_ab) instead of read from slot tau, which it writes
-void launch_friction_ab(Model &m, int itt, int tau, int taum1, int taum2, bool with_tendency = false);
+void launch_friction_ab(Model &m, int itt, int tau, int taum1, int taum2);
 void launch_border_exchg(Model &m, double *a, int neumann_z);
 void launch_project_exchange(Model &m);
 
@@ -337,9 +330,10 @@ void tridiag_factor(Model &m);
 void launch_thomas(Model &m, double2 *data);
 void launch_thomas_f(Model &m, float2 *data);
 
-void launch_friction_ab_raw(Model &m, int itt, int tau, int taum1, int taum2, bool with_tendency = false);
-// the step takes k_tend_fric_ab (tendency, friction and AB in one kernel)
-bool fused_tendency_active(const Model &m);
+// levels per work-group of the k-marching kernels when not tuned: tiles
+// column tiles march together over nz levels
+int friction_levels(int tiles, int nz, bool mixed);
+void launch_friction_ab_raw(Model &m, int itt, int tau, int taum1, int taum2);
 // forced FP64 step: the fused friction chain alone into the second buffers
 // (halos pre-friction), marked current for the forcing and launch_ab_exchange
 void launch_friction_fused_only(Model &m);

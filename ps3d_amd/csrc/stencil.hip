@@ -10,6 +10,7 @@
 // instead of one per flux array.
 #include "ps3d_internal.h"
 
+#include <algorithm>
 #include <type_traits>
 
 #pragma clang fp contract(off)
@@ -720,11 +721,35 @@ __global__ __launch_bounds__(BX * BY) void k_background_ab(StepConsts c, BgArgs<
 // points keep f0, as in the reference); each tile point then applies
 // biharmonic_h to f1 and the AB update, writing a second buffer (neighbouring
 // tiles still read f0).
+//
+// Bound: memory, once enough of a CU's wavefronts are ready to issue.  A
+// plane comes in by one 16-byte direct-to-LDS load per lane, two levels ahead
+// of its use, instead of two loads to registers and two LDS writes: a tenth
+// fewer vector instructions, and 62 instead of 72 vector registers, so that
+// four work-groups fit a CU.  FP64, 256x256x64: 152 -> 131 us, 765 MB of
+// traffic (671 compulsory) at 5.8 TB/s, the rate of a streaming copy;
+// 512x512x64 672 -> 590 us; 1024x1024x128 5.77 -> 5.01 ms.  Mixed,
+// 256x256x64: 144 -> 137 us (79 registers, three work-groups per CU; at 64
+// registers it spills and takes 190 us).
 // ---------------------------------------------------------------------------
 constexpr int FTX = FRIC_TX, FTY = FRIC_TY;
-constexpr int R0X = FTX + 6, R0Y = FTY + 6;
 constexpr int R1X = FTX + 4, R1Y = FTY + 4;
 constexpr int FTHREADS = FTX * FTY;
+
+// f0 planes in LDS: the tile and its 3-point apron, rows widened to whole
+// 16-byte chunks that are aligned in memory (a field's row starts at a
+// multiple of 16 bytes and holds i at element i + 1, a tile starts at i =
+// 64 m + 1), so that one direct-to-LDS load per lane brings in a plane
+template <class T>
+struct FricPlane {
+    static constexpr int CH = 16 / (int)sizeof(T);          // values per chunk
+    static constexpr int OX = sizeof(T) == 8 ? 4 : 6;       // columns before the tile
+    static constexpr int W = (OX + FTX + 3 + CH - 1) / CH * CH;
+    static constexpr int ROWS = FTY + 6;
+    static constexpr int N = W * ROWS, NCH = N / CH;
+    static_assert(NCH <= FTHREADS, "one chunk per lane");
+    static constexpr int WAVES = sizeof(T) == 8 ? 1 : 6;    // least per SIMD, for the register allocation
+};
 
 template <class T>
 struct FricField {
@@ -762,65 +787,26 @@ __device__ __forceinline__ int fric_field(const FricArgs<T> &a, int bid)
     return bid / (a.tiles_x * a.tiles_y) / a.nchunk;
 }
 
-// The tendency fused in (TF = 0..3, the field of the work-group, FP64 only):
-// the work-group forms field TF's tendency at its tile points (the
-// expressions of tendency_fp64) from its own ring of f0 and, for the other
-// fields, values loaded from global memory at the few points the stencil
-// reads -- the work-groups of the same tile and chunk that own those fields
-// run next to it on the same XCD and bring them into L2.  The tendency goes
-// straight into the AB sum and into slot tau, which is never read back.
-template <int TF, class A>
-__device__ __forceinline__ double fused_tendency(const StepConsts &c, int k, A ring, const double *e0,
-                                                 const double *em, const double *ep)
+// one 16-byte (or 4-byte) direct-to-LDS load per lane: global address per
+// lane, LDS address lds + lane * BYTES (lds uniform in the wavefront)
+template <int BYTES>
+__device__ __forceinline__ void load_to_lds(const void *g, void *lds)
 {
-    auto F = [&](int f, int dk, int dj, int di) -> double {
-        if (f == TF) return ring(dk, dj, di);
-        if constexpr (TF == 0) {   // V at k: (j, i+1), (j, i), (j-1, i+1), (j-1, i); W at k, k-1: (j, i), (j, i+1)
-            if (f == 1) return e0[(dj == 0 ? 0 : 2) + (di == 1 ? 0 : 1)];
-            return dk == 0 ? e0[4 + di] : em[di];
-        } else if constexpr (TF == 1) {   // U at k: (j+1, i), (j, i), (j+1, i-1), (j, i-1); W at k, k-1: (j, i), (j+1, i)
-            if (f == 0) return e0[(di == 0 ? 0 : 2) + (dj == 1 ? 0 : 1)];
-            return dk == 0 ? e0[4 + dj] : em[dj];
-        } else if constexpr (TF == 2) {   // at k and k+1: U (j, i), (j, i-1); V (j, i), (j-1, i); B (j, i)
-            const double *e = dk == 0 ? e0 : ep;
-            if (f == 0) return e[di == 0 ? 0 : 1];
-            if (f == 1) return e[2 + (dj == 0 ? 0 : 1)];
-            return e[4];
-        } else {   // U at k: (j, i), (j, i-1); V at k: (j, i), (j-1, i); W at k, k-1: (j, i)
-            if (f == 0) return e0[di == 0 ? 0 : 1];
-            if (f == 1) return e0[2 + (dj == 0 ? 0 : 1)];
-            return dk == 0 ? e0[4] : em[0];
-        }
-    };
-    return tendency_fp64<TF>(c, k, F);
+    const auto *gp = (const __attribute__((address_space(1))) void *)g;
+    auto *lp = (__attribute__((address_space(3))) void *)lds;
+    if constexpr (BYTES == 16) __builtin_amdgcn_global_load_lds(gp, lp, 16, 0, 0);
+    else __builtin_amdgcn_global_load_lds(gp, lp, 4, 0, 0);
 }
 
-// the other fields' values of fused_tendency<TF> at level kk (see there)
-template <int TF>
-__device__ __forceinline__ void fused_tendency_load(const StepConsts &c, const FricArgs<double> &a, int i, int j,
-                                                    int kk, double *e)
-{
-    const int64_t o = (int64_t)(i + 1) + c.X * (int64_t)(j + 1) + c.XY * (int64_t)(kk + 1);
-    const int64_t X = c.X;
-    const double *U = a.f[0].in, *V = a.f[1].in, *W = a.f[2].in, *B = a.f[3].in;
-    if constexpr (TF == 0) {
-        e[0] = V[o + 1]; e[1] = V[o]; e[2] = V[o + 1 - X]; e[3] = V[o - X]; e[4] = W[o]; e[5] = W[o + 1];
-    } else if constexpr (TF == 1) {
-        e[0] = U[o + X]; e[1] = U[o]; e[2] = U[o + X - 1]; e[3] = U[o - 1]; e[4] = W[o]; e[5] = W[o + X];
-    } else if constexpr (TF == 2) {
-        e[0] = U[o]; e[1] = U[o - 1]; e[2] = V[o]; e[3] = V[o - X]; e[4] = B[o];
-    } else {
-        e[0] = U[o]; e[1] = U[o - 1]; e[2] = V[o]; e[3] = V[o - X]; e[4] = W[o];
-    }
-}
-
-template <class T, int TF = -1>
+template <class T>
 __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T> &a, const FricField<T> &F, int bid)
 {
-    static_assert(TF < 0 || std::is_same<T, double>::value, "the fused tendency is FP64 only");
-    constexpr bool TEND = TF >= 0;
     constexpr bool MIXED = std::is_same<T, float>::value;
-    __shared__ T f0p[3][R0Y][R0X];
+    using PL = FricPlane<T>;
+    constexpr int W = PL::W, OX = PL::OX, CH = PL::CH;
+    // f0 of three levels.  Three arrays, not one: the compiler then knows
+    // that reads of one need not wait for loads into another.
+    __shared__ __attribute__((aligned(16))) T pl0[PL::N], pl1[PL::N], pl2[PL::N];
     __shared__ T f1p[R1Y][R1X];
     __shared__ T d2p[FTY + 2][FTX + 2];   // biharmonic_h's del2 on the tile + 1
     __shared__ T hinc[MIXED ? FTY : 1][MIXED ? FTX : 1];   // harmonic increment at tile points
@@ -833,43 +819,39 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
     const int kb = 1 + ch * a.kc;
     const int ke = min(c.nz, kb + a.kc - 1);
     const int t = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int nx = c.nx, ny = c.ny, nz = c.nz;
     const bool lid = c.lid != 0;
     const double dx = c.dx, dy = c.dy, dz = c.dz, rdx = c.rdx, rdy = c.rdy, rdz = c.rdz;
     const T dt = (T)c.dt;
     const T zero = T(0);
 
-    auto slot = [&](int k) { return (k - kb + 1) % 3; };
-    constexpr int PER = (R0X * R0Y + FTHREADS - 1) / FTHREADS;
-    T pre[PER];
-    auto fetch = [&](int k) {
-#pragma unroll
-        for (int s = 0; s < PER; ++s) {
-            const int q = t + s * FTHREADS;
-            const int rx = q % R0X, ry = q / R0X;
-            const int ii = i0 - 3 + rx, jj = j0 - 3 + ry;
-            const bool ok = q < R0X * R0Y && ii >= -1 && ii <= nx + 2 && jj >= -1 && jj <= ny + 2;
-            pre[s] = ok ? F.in[idx(c, ii, jj, k)] : zero;
-        }
+    // loads of a plane: rows past the array's are clamped, columns past a
+    // row's ends run into the rows beside (in the array: a level lies on
+    // either side); neither enters a stored value
+    const bool chunks = sizeof(T) == 8 || c.X % CH == 0;   // rows start at 16-byte boundaries
+    auto src = [&](int q) {   // element q of the plane, from the level's start
+        const int jj = min(max(j0 - 3 + q / W, -1), ny + 2);
+        return (int64_t)(i0 - OX + 1 + q % W) + c.X * (int64_t)(jj + 1);
     };
-    auto store = [&](int k) {
-        const int sl = slot(k);
-#pragma unroll
-        for (int s = 0; s < PER; ++s) {
-            const int q = t + s * FTHREADS;
-            if (q < R0X * R0Y) f0p[sl][q / R0X][q % R0X] = pre[s];
+    const T *mysrc = F.in + src(t < PL::NCH ? t * CH : 0);
+    auto fetch = [&](T *dst, int k) {
+        const int64_t lk = c.XY * (int64_t)(k + 1);
+        if (chunks) {
+            if (t < PL::NCH) load_to_lds<16>(mysrc + lk, dst + wave * 64 * CH);
+        } else {
+            for (int s = 0; s * FTHREADS < PL::N; ++s) {
+                const int q = t + s * FTHREADS;
+                if (q < PL::N) load_to_lds<4>(F.in + src(q) + lk, dst + s * FTHREADS + wave * 64);
+            }
         }
     };
     const int tpx = t % FTX, tpy = t / FTX;
     const bool mine = (i0 + tpx <= nx) && (j0 + tpy <= ny);
 
-    fetch(kb - 1);
-    store(kb - 1);
-    fetch(kb);
-    store(kb);
-    fetch(kb + 1);
-    // the tendency slots (and lo part) of a level are loaded one level ahead,
-    // so their latency overlaps a whole level's LDS phases
+    // the tendency slots (and lo part) of a level at the lane's point, read
+    // once: streamed past the L2, which keeps the f0 planes that
+    // neighbouring tiles share
     struct Pt {
         T s0, s1, s2, lo0;
         float q1o, q1n, q2o, q2n;   // mixed form: pressure-history increments
@@ -878,9 +860,7 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
         Pt r{zero, zero, zero, zero, 0.f, 0.f, 0.f, 0.f};
         if (mine) {
             const int64_t o = idx(c, i0 + tpx, j0 + tpy, k);
-            // read once: streamed past the L2, which keeps the f0 planes
-            // that neighbouring tiles share
-            if constexpr (!TEND) r.s0 = __builtin_nontemporal_load(F.t0 + o);
+            if (a.order >= 1) r.s0 = __builtin_nontemporal_load(F.t0 + o);
             if (a.order >= 2) r.s1 = __builtin_nontemporal_load(F.t1 + o);
             if (a.order >= 3) r.s2 = __builtin_nontemporal_load(F.t2 + o);
             if constexpr (MIXED) {
@@ -897,66 +877,51 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
         }
         return r;
     };
-    Pt nxt = load_pt(kb);
+
     // harmonic: the vertical flux through each point's upper face, for the
-    // next level's lower face
+    // next level's lower face (the same operands, so the same bits); a thread
+    // keeps its points from level to level
     constexpr int NSQ1 = (R1X * R1Y + FTHREADS - 1) / FTHREADS;
     T ftc[NSQ1];
+
+    fetch(pl0, kb - 1);
+    fetch(pl1, kb);
+    fetch(pl2, kb + 1);
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+    __syncthreads();
 #pragma unroll
-    for (int sq = 0; sq < NSQ1; ++sq) ftc[sq] = zero;
-    // fused tendency: the other fields' values at level k (e0), k - 1 (em:
-    // W, carried from the level before) and k + 1 (ep, field w only)
-    double e0[6] = {}, em[2] = {}, ep[6] = {};
-    if constexpr (TEND) {
-        if (mine) {
-            if constexpr (TF == 2) fused_tendency_load<TF>(c, a, i0 + tpx, j0 + tpy, kb, ep);
-            else fused_tendency_load<TF>(c, a, i0 + tpx, j0 + tpy, kb - 1, e0);
+    for (int sq = 0; sq < NSQ1; ++sq) {
+        const int q = t + sq * FTHREADS;
+        ftc[sq] = zero;
+        if (q < R1X * R1Y && !(lid && kb - 1 <= 0)) {
+            const int o = (q / R1X + 1) * W + q % R1X + OX - 2;
+            ftc[sq] = sdiv<T>((T)F.Vm * (pl1[o] - pl0[o]), dz, rdz);
         }
     }
-    for (int k = kb; k <= ke; ++k) {
-        store(k + 1);
-        if (k + 1 <= ke) fetch(k + 2);
-        const Pt cur = nxt;
-        if (k + 1 <= ke) nxt = load_pt(k + 1);
-        if constexpr (TEND) {
-            if (mine) {
-                if constexpr (TF == 2) {
-#pragma unroll
-                    for (int q = 0; q < 6; ++q) e0[q] = ep[q];
-                    fused_tendency_load<TF>(c, a, i0 + tpx, j0 + tpy, k + 1, ep);
-                } else {
-                    if constexpr (TF == 3) em[0] = e0[4];
-                    else { em[0] = e0[4]; em[1] = e0[5]; }
-                    fused_tendency_load<TF>(c, a, i0 + tpx, j0 + tpy, k, e0);
-                }
-            }
-        }
-        const T s0 = cur.s0, s1 = cur.s1, s2 = cur.s2, lo0 = cur.lo0;
-        const float q1o = cur.q1o, q1n = cur.q1n, q2o = cur.q2o, q2n = cur.q2n;
+
+    // level k: f0 of levels k and k + 1 in sc and sp, that of level k + 2
+    // fetched into sn meanwhile
+    auto level = [&](int k, const T *sc, const T *sp, T *sn) {
         __syncthreads();
-        const int sm = slot(k - 1), sc = slot(k), sp = slot(k + 1);
+        if (k + 1 <= ke) fetch(sn, k + 2);
+        const Pt cur = load_pt(k);
 #pragma unroll
         for (int sq = 0; sq < NSQ1; ++sq) {
             const int q = t + sq * FTHREADS;
             if (q >= R1X * R1Y) break;
             const int rx = q % R1X, ry = q / R1X;
             const int ii = i0 - 2 + rx, jj = j0 - 2 + ry;
-            const int ox = rx + 1, oy = ry + 1;
-            const T v0 = f0p[sc][oy][ox];
+            const int o = (ry + 1) * W + rx + OX - 2;
+            const T v0 = sc[o];
             T f1 = v0, inc = zero;
             if (F.harm && ii >= 1 && ii <= nx && jj >= 1 && jj <= ny) {
                 const T Hm = (T)F.Hm, Vm = (T)F.Vm;
-                const T fe1 = sdiv<T>(Hm * (f0p[sc][oy][ox + 1] - v0), dx, rdx);
-                const T fe0 = sdiv<T>(Hm * (v0 - f0p[sc][oy][ox - 1]), dx, rdx);
-                const T fn1 = sdiv<T>(Hm * (f0p[sc][oy + 1][ox] - v0), dy, rdy);
-                const T fn0 = sdiv<T>(Hm * (v0 - f0p[sc][oy - 1][ox]), dy, rdy);
-                const T ft1 = (lid && k >= nz) ? zero : sdiv<T>(Vm * (f0p[sp][oy][ox] - v0), dz, rdz);
-                // the flux through the face below is the face above of the
-                // level before (the same operands, so the same bits), carried
-                // by the thread, which keeps its point from level to level;
-                // formed here at the chunk's first level
-                const T ft0 = k > kb ? ftc[sq]
-                                     : ((lid && k - 1 <= 0) ? zero : sdiv<T>(Vm * (v0 - f0p[sm][oy][ox]), dz, rdz));
+                const T fe1 = sdiv<T>(Hm * (sc[o + 1] - v0), dx, rdx);
+                const T fe0 = sdiv<T>(Hm * (v0 - sc[o - 1]), dx, rdx);
+                const T fn1 = sdiv<T>(Hm * (sc[o + W] - v0), dy, rdy);
+                const T fn0 = sdiv<T>(Hm * (v0 - sc[o - W]), dy, rdy);
+                const T ft1 = (lid && k >= nz) ? zero : sdiv<T>(Vm * (sp[o] - v0), dz, rdz);
+                const T ft0 = ftc[sq];
                 ftc[sq] = ft1;
                 inc = dt * (sdiv<T>(fe1 - fe0, dx, rdx) + sdiv<T>(fn1 - fn0, dy, rdy) + sdiv<T>(ft1 - ft0, dz, rdz));
                 f1 = v0 + inc;
@@ -982,6 +947,9 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
             }
             __syncthreads();
         }
+        // the next plane has arrived before this level's stores begin, so the
+        // wait is never for them
+        __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
         if (mine) {
             const int px = tpx, py = tpy;
             const int i = i0 + px, j = j0 + py;
@@ -998,43 +966,31 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
             }
             const int64_t o = idx(c, i, j, k);
             if constexpr (!MIXED) {
-                double s0t = s0;
-                if constexpr (TEND) {
-                    const int sm2 = slot(k - 1), sc2 = slot(k), sp2 = slot(k + 1);
-                    const int ry0 = py + 3, rx0 = px + 3;
-                    auto ring = [&](int dk, int dj, int di) -> double {
-                        const int sl = dk < 0 ? sm2 : (dk > 0 ? sp2 : sc2);
-                        return f0p[sl][ry0 + dj][rx0 + di];
-                    };
-                    s0t = fused_tendency<TF>(c, k, ring, e0, em, ep);
-                    // slot tau (read-only elsewhere in this kernel), for the next steps' AB sums
-                    const_cast<double *>(F.t0)[o] = s0t;
-                }
                 const double s = F.scale;
                 double val;
                 if (a.order == 0) val = f2;   // friction only (the split step of a forced model)
-                else if (a.order == 1) val = f2 + s * s0t;
-                else if (a.order == 2) val = f2 + s * (a.ca * s0t - a.cb * s1);
-                else val = f2 + s * (a.ca * s0t + a.cb * s1 + a.cc * s2);
+                else if (a.order == 1) val = f2 + s * cur.s0;
+                else if (a.order == 2) val = f2 + s * (a.ca * cur.s0 - a.cb * cur.s1);
+                else val = f2 + s * (a.ca * cur.s0 + a.cb * cur.s1 + a.cc * cur.s2);
                 F.out[o] = val;
                 if (a.halo) write_images<double>(c, F.out, i, j, k, val, 0);
             } else {
                 const double s = F.scale;
                 double ab;
                 if (a.order == 0) ab = 0.0;   // friction only (the split step of a forced mixed model)
-                else if (a.order == 1) ab = s * (double)s0;
-                else if (a.order == 2) ab = s * (a.ca * (double)s0 - a.cb * (double)s1);
-                else ab = s * (a.ca * (double)s0 + a.cb * (double)s1 + a.cc * (double)s2);
+                else if (a.order == 1) ab = s * (double)cur.s0;
+                else if (a.order == 2) ab = s * (a.ca * (double)cur.s0 - a.cb * (double)cur.s1);
+                else ab = s * (a.ca * (double)cur.s0 + a.cb * (double)cur.s1 + a.cc * (double)cur.s2);
                 // the harmonic pass zeroes w(nz) under a rigid lid before the
                 // biharmonic and AB increments are added
                 const bool zt = F.zero_top && k >= nz;
-                const double base = zt ? 0.0 : (double)f0p[sc][cy + 1][cx + 1] + (double)lo0;
+                const double base = zt ? 0.0 : (double)sc[(cy + 1) * W + px + OX] + (double)cur.lo0;
                 double gq = 0.0;
                 if (F.gstride && a.d1) {
-                    double qo = a.qc1 * (double)q1o, qn = a.qc1 * (double)q1n;
+                    double qo = a.qc1 * (double)cur.q1o, qn = a.qc1 * (double)cur.q1n;
                     if (a.d2) {
-                        qo += a.qc2 * (double)q2o;
-                        qn += a.qc2 * (double)q2n;
+                        qo += a.qc2 * (double)cur.q2o;
+                        qn += a.qc2 * (double)cur.q2n;
                     }
                     gq = F.scale * ((qn - qo) * F.grd);
                 }
@@ -1046,31 +1002,23 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
             }
         }
         // no barrier here: the next level's first barrier orders this level's
-        // reads of f1p, d2p and hinc before their next writes, and the f0p
-        // slot refilled next held level k-2, last read before this level's
-        // second barrier
+        // reads of f1p, d2p, hinc and sc before their next writes
+    };
+    for (int k = kb;;) {
+        level(k, pl1, pl2, pl0);
+        if (++k > ke) break;
+        level(k, pl2, pl0, pl1);
+        if (++k > ke) break;
+        level(k, pl0, pl1, pl2);
+        if (++k > ke) break;
     }
 }
 
 template <class T>
-__global__ __launch_bounds__(FTHREADS) void k_fric_ab(StepConsts c, FricArgs<T> a)
+__global__ __launch_bounds__(FTHREADS, FricPlane<T>::WAVES) void k_fric_ab(StepConsts c, FricArgs<T> a)
 {
     const int bid = xcd_remap((int)blockIdx.x, a.nblocks);
     fric_body<T>(c, a, a.f[fric_field(a, bid)], bid);
-}
-
-// tendency (integrate.f90:12-54), friction chain and Adams-Bashforth of the
-// four fields in one launch (FP64): blocks run over (field, tile, chunk) with
-// the field fastest, so the four work-groups of a tile and chunk sit together
-// on one XCD and share the state's planes in its L2
-__global__ __launch_bounds__(FTHREADS) void k_tend_fric_ab(StepConsts c, FricArgs<double> a)
-{
-    const int bid = xcd_remap((int)blockIdx.x, a.nblocks);
-    const int f = bid & 3, rest = bid >> 2;
-    if (f == 0) fric_body<double, 0>(c, a, a.f[0], rest);
-    else if (f == 1) fric_body<double, 1>(c, a, a.f[1], rest);
-    else if (f == 2) fric_body<double, 2>(c, a, a.f[2], rest);
-    else fric_body<double, 3>(c, a, a.f[3], rest);
 }
 
 // ---------------------------------------------------------------------------
@@ -1323,7 +1271,7 @@ __global__ __launch_bounds__(TTHR) void k_ens_tendency(const EnsMember *__restri
     tendency_body<double>(c, a, g - map.start[mi]);
 }
 
-__global__ __launch_bounds__(FTHREADS) void k_ens_fric(const EnsMember *__restrict__ mem, EnsMap map,
+__global__ __launch_bounds__(FTHREADS, FricPlane<double>::WAVES) void k_ens_fric(const EnsMember *__restrict__ mem, EnsMap map,
                                                         const EnsState *__restrict__ st)
 {
     const int g = xcd_remap((int)blockIdx.x, map.start[map.n]);
@@ -1619,7 +1567,7 @@ __global__ __launch_bounds__(TTHR) void k_ens_tendency_f(const EnsMember *__rest
     tendency_body<float>(c, a, g - map.start[mi]);
 }
 
-__global__ __launch_bounds__(FTHREADS) void k_ens_fric_f(const EnsMember *__restrict__ mem, EnsMap map,
+__global__ __launch_bounds__(FTHREADS, FricPlane<float>::WAVES) void k_ens_fric_f(const EnsMember *__restrict__ mem, EnsMap map,
                                                           const EnsState *__restrict__ st, int cold)
 {
     const int g = xcd_remap((int)blockIdx.x, map.start[map.n]);
@@ -1775,6 +1723,21 @@ inline dim3 march_grid(const Grid &g, int &kc)
     kc = kc < 4 ? (g.nz < 4 ? g.nz : 4) : kc;
     nch = (g.nz + kc - 1) / kc;
     return dim3((unsigned)((g.nx + BX - 1) / BX), (unsigned)((g.ny + BY - 1) / BY), (unsigned)nch);
+}
+
+// Levels per work-group of the friction kernel: at least 1024 work-groups
+// (four per CU), of 2 to 8 levels (mixed form: to 16).  Short chunks keep the
+// tiles that share apron rows within reach of one L2: FP64, 512x512x64, 590
+// us with 8 levels, 617 with 16, 650 with 32, 683 with 64; 256x256x64, 131
+// with 8 or 16, 155 with 32.  Below 2 levels the three planes that a chunk
+// reads before its first level cost more than the work-groups give (64x64x32:
+// 13.2 us with 2, 14.4 with 1 or 4).  Mixed, 256x256x64: 137 us with 16, 144
+// with 8.
+int friction_levels(int tiles, int nz, bool mixed)
+{
+    const int most = mixed ? 16 : 8;
+    const int nchunk = std::max((nz + most - 1) / most, (1024 + 4 * tiles - 1) / (4 * tiles));
+    return std::max(std::min(nz, 2), (nz + nchunk - 1) / nchunk);
 }
 
 template <class T>
@@ -2039,13 +2002,6 @@ bool fused_friction_ok(const Model &m)
     return !(m.prm.Avbi > 0.) && !(m.prm.Kvbi > 0.);
 }
 
-bool fused_tendency_active(const Model &m)
-{
-    const bool forced = m.forcing || m.wm_on || m.bg_on ||
-                        (m.bf_on[0] || m.bf_on[1] || m.bf_on[2] || m.bf_on[3]);
-    return !m.mixed && fused_friction_ok(m) && m.fuse_friction && m.fuse_tendency && !forced;
-}
-
 // integrate.f90:59-111 for configs without vertical biharmonic friction:
 // the friction chain and AB of all four fields in one launch, which also
 // writes the new values' halo images (the exchange of integrate.f90:106-111).
@@ -2056,8 +2012,7 @@ bool fused_tendency_active(const Model &m)
 template <class T>
 static void friction_ab_impl(Model &m, const T *const *in, const T *const *in_lo, T *const *out, T *const *out_lo,
                              T *const *tend, int itt, int tau, int taum1, int taum2, double qc1 = 0.0,
-                             const float *d1 = nullptr, double qc2 = 0.0, const float *d2 = nullptr, int halo = -1,
-                             bool fuse_tend = false)
+                             const float *d1 = nullptr, double qc2 = 0.0, const float *d2 = nullptr, int halo = -1)
 {
     const ps3d_params &p = m.prm;
     const Grid &g = m.g;
@@ -2110,25 +2065,10 @@ static void friction_ab_impl(Model &m, const T *const *in, const T *const *in_lo
     a.tiles_x = (g.nx + FTX - 1) / FTX;
     a.tiles_y = (g.ny + FTY - 1) / FTY;
     const int tiles = a.tiles_x * a.tiles_y;
-    const int target = 2048 * 512 / FTHREADS;   // ~8 work-groups of 512 threads per CU
-    int nchunk = (target + tiles * 4 - 1) / (tiles * 4);
-    nchunk = nchunk < 1 ? 1 : (nchunk > g.nz ? g.nz : nchunk);
-    const int kc_set = fuse_tend ? m.tfric_kc : m.fric_kc;
-    if (kc_set > 0) nchunk = (g.nz + kc_set - 1) / kc_set;
-    a.kc = (g.nz + nchunk - 1) / nchunk;
+    a.kc = m.fric_kc > 0 ? m.fric_kc : friction_levels(tiles, g.nz, std::is_same<T, float>::value);
     a.nchunk = (g.nz + a.kc - 1) / a.kc;
     a.nblocks = tiles * a.nchunk * 4;
     a.halo = halo < 0 ? (m.fuse_halo ? 1 : 0) : halo;
-    if constexpr (std::is_same<T, double>::value) {
-        if (fuse_tend) {
-            PS3D_REQUIRE(itt >= 0, "tendency + friction + AB: itt >= 0");
-            ProfScope ps(m, "tend_friction_ab");
-            hipLaunchKernelGGL(k_tend_fric_ab, dim3((unsigned)a.nblocks), dim3(FTHREADS), 0, m.stream, m.c, a);
-            PS3D_HIP_CHECK(hipGetLastError());
-            return;
-        }
-    }
-    PS3D_REQUIRE(!fuse_tend, "tendency + friction + AB: FP64 models only");
     ProfScope ps(m, "friction_ab");
     hipLaunchKernelGGL(k_fric_ab<T>, dim3((unsigned)a.nblocks), dim3(FTHREADS), 0, m.stream, m.c, a);
     PS3D_HIP_CHECK(hipGetLastError());
@@ -2254,7 +2194,7 @@ void launch_friction_fused_only(Model &m)
     for (int f = 0; f < 4; ++f) m.cur[f] = 1;
 }
 
-void launch_friction_ab_raw(Model &m, int itt, int tau, int taum1, int taum2, bool with_tendency)
+void launch_friction_ab_raw(Model &m, int itt, int tau, int taum1, int taum2)
 {
     if (m.mixed) {
         launch_friction_ab_mixed(m, itt, tau, taum1, taum2, 0.0, nullptr, 0.0, nullptr, false);
@@ -2262,17 +2202,15 @@ void launch_friction_ab_raw(Model &m, int itt, int tau, int taum1, int taum2, bo
     }
     double *in[4] = {m.u, m.v, m.w, m.b};
     double *tend[4] = {m.du, m.dv, m.dw, m.db};
-    friction_ab_impl<double>(m, in, nullptr, m.alt, nullptr, tend, itt, tau, taum1, taum2, 0.0, nullptr, 0.0,
-                             nullptr, -1, with_tendency);
+    friction_ab_impl<double>(m, in, nullptr, m.alt, nullptr, tend, itt, tau, taum1, taum2);
 }
 
-void launch_friction_ab(Model &m, int itt, int tau, int taum1, int taum2, bool with_tendency)
+void launch_friction_ab(Model &m, int itt, int tau, int taum1, int taum2)
 {
     PS3D_REQUIRE(!m.mixed, "friction_ab: FP64 models only");
     double *in[4] = {m.u, m.v, m.w, m.b};
     double *tend[4] = {m.du, m.dv, m.dw, m.db};
-    friction_ab_impl<double>(m, in, nullptr, m.alt, nullptr, tend, itt, tau, taum1, taum2, 0.0, nullptr, 0.0,
-                             nullptr, -1, with_tendency);
+    friction_ab_impl<double>(m, in, nullptr, m.alt, nullptr, tend, itt, tau, taum1, taum2);
     std::swap(m.u, m.alt[0]);
     std::swap(m.v, m.alt[1]);
     std::swap(m.w, m.alt[2]);

@@ -182,20 +182,13 @@ void tune_model(Model &m, int next_tau, const char *cache_path, int reps)
         cache[key] = best;
     };
 
-    if (fused_tendency_active(m)) {
-        // the fused kernel writes slot next_tau (overwritten by the next
-        // step) and the second buffers
-        pick("tend_friction_ab", levels, m.tfric_kc, reps, nullptr,
-             [&] { launch_friction_ab_raw(m, 3, next_tau, t1, t2, true); });
-    } else {
-        pick("tendency", levels, m.tend_kc, reps, nullptr, [&] {
-            if (m.mixed) launch_tendency_mixed(m, next_tau, m.pint);
-            else launch_tendency(m, next_tau);
-        });
-        if (m.mixed || (fused_friction_ok(m) && m.fuse_friction))
-            pick("friction_ab", levels, m.fric_kc, reps, nullptr,
-                 [&] { launch_friction_ab_raw(m, 3, next_tau, t1, t2); });
-    }
+    pick("tendency", levels, m.tend_kc, reps, nullptr, [&] {
+        if (m.mixed) launch_tendency_mixed(m, next_tau, m.pint);
+        else launch_tendency(m, next_tau);
+    });
+    if (m.mixed || (fused_friction_ok(m) && m.fuse_friction))
+        pick("friction_ab", levels, m.fric_kc, reps, nullptr,
+             [&] { launch_friction_ab_raw(m, 3, next_tau, t1, t2); });
     if (m.mixed) {
         // radix plans of the FP32 transforms, on scratch arrays: the forward
         // x pass reads the state and writes the scratch spectrum, the other
@@ -288,12 +281,8 @@ std::string describe_tuning(const Model &m)
 {
     std::ostringstream o;
     const std::string sh = shape_of(m);
-    if (fused_tendency_active(m)) {
-        o << "tend_friction_ab " << sh << " " << m.tfric_kc << "\n";
-    } else {
-        o << "tendency " << sh << " " << m.tend_kc << "\n";
-        o << "friction_ab " << sh << " " << m.fric_kc << "\n";
-    }
+    o << "tendency " << sh << " " << m.tend_kc << "\n";
+    o << "friction_ab " << sh << " " << m.fric_kc << "\n";
     o << "thomas " << sh << " " << m.thomas_cpw << "\n";
     if (m.mixed) {
         const char *names[3] = {"fft_plan_x", "fft_plan_y", "fft_plan_z"};

@@ -283,8 +283,8 @@ class Model:
         check(self.lib.ps3d_set_forcing(self.h, ctypes.cast(self._forcing_cb, ctypes.c_void_p), None))
 
     def set_fused_tendency(self, on: bool):
-        """Form the tendencies inside the friction + AB kernel (True) or in a
-        kernel of their own (False, the default): ps3d_set_fused_tendency."""
+        """Accepted; both settings run the same kernels
+        (ps3d_set_fused_tendency)."""
         check(self.lib.ps3d_set_fused_tendency(self.h, 1 if on else 0))
 
     @property
