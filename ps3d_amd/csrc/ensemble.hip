@@ -73,24 +73,6 @@ void set_chunks(int nz, int kc, int &okc, int &onch)
     okc = cdiv(nz, onch);
 }
 
-// the single-model launchers' choices (stencil.hip), the untuned default
-int default_tend_kc(const Grid &g)
-{
-    const int tiles = cdiv(g.nx, kTTX) * cdiv(g.ny, kTTY);
-    int nchunk = cdiv(512, tiles);
-    const int maxch = g.nz / 8 > 1 ? g.nz / 8 : 1;
-    nchunk = std::min(nchunk, maxch);
-    return cdiv(g.nz, nchunk);
-}
-
-int default_fric_kc(const Grid &g)
-{
-    const int tiles = cdiv(g.nx, kFTX) * cdiv(g.ny, kFTY);
-    int nchunk = cdiv(2048 * 512 / (kFTX * kFTY), tiles * 4);
-    nchunk = std::max(1, std::min(nchunk, g.nz));
-    return cdiv(g.nz, nchunk);
-}
-
 void fill_member(EnsMember &e, ps3d_model &m)
 {
     const ps3d_params &p = m.prm;
@@ -539,8 +521,17 @@ int ps3d_ensemble_create(int n, const ps3d_params *prms, void *stream, ps3d_ense
                 if (rc != PS3D_OK) throw Error(rc, "member " + std::to_string(i) + ": " + error_slot());
                 E->mem[i] = m;
                 fill_member(E->tab[i], *m);
-                set_chunks(m->g.nz, default_tend_kc(m->g), E->tab[i].tend_kc, E->tab[i].tend_nchunk);
-                set_chunks(m->g.nz, default_fric_kc(m->g), E->tab[i].fric_kc, E->tab[i].fric_nchunk);
+            }
+            // untuned levels per work-group: those of a single model with the
+            // tiles of all members, which march together
+            int ttiles = 0, ftiles = 0;
+            for (const EnsMember &e : E->tab) {
+                ttiles += e.tend_tx * e.tend_ty;
+                ftiles += e.fric_tx * e.fric_ty;
+            }
+            for (EnsMember &e : E->tab) {
+                set_chunks(e.c.nz, tendency_levels(ttiles, e.c.nz), e.tend_kc, e.tend_nchunk);
+                set_chunks(e.c.nz, friction_levels(ftiles, e.c.nz, E->mixed), e.fric_kc, e.fric_nchunk);
             }
             bool reg = true, split = true;
             for (ps3d_model *m : E->mem)

@@ -1725,6 +1725,18 @@ inline dim3 march_grid(const Grid &g, int &kc)
     return dim3((unsigned)((g.nx + BX - 1) / BX), (unsigned)((g.ny + BY - 1) / BY), (unsigned)nch);
 }
 
+// Levels per work-group of the tendency kernel: at least 512 work-groups (two
+// per CU) where the grid has the levels for it, of at most 16 levels.  On
+// small grids a work-group's levels are one after the other on an idle chip:
+// 64x64x32, 9.6 us with 1 level, 14.5 with 4, 21.9 with 8; 120x120x10, 10.7
+// with 1, 25 with 10; 160x120x37, 20 with 4, 31 with 13.  On large ones
+// 512x512x64 takes 250 us with 16 levels, 262 with 64.
+int tendency_levels(int tiles, int nz)
+{
+    const int nchunk = std::min(nz, std::max((nz + 15) / 16, (512 + tiles - 1) / tiles));
+    return (nz + nchunk - 1) / nchunk;
+}
+
 // Levels per work-group of the friction kernel: at least 1024 work-groups
 // (four per CU), of 2 to 8 levels (mixed form: to 16).  Short chunks keep the
 // tiles that share apron rows within reach of one L2: FP64, 512x512x64, 590
@@ -1755,14 +1767,7 @@ static void tendency_impl(Model &m, const T *u, const T *v, const T *w, const T 
     a.tiles_x = (g.nx + TTX - 1) / TTX;
     a.tiles_y = (g.ny + TTY - 1) / TTY;
     const int tiles = a.tiles_x * a.tiles_y;
-    // about 2 work-groups per CU over 256 CUs, chunks of at least 8 levels
-    // (or the tuned number of levels): longer chunks re-read fewer apron
-    // planes, which at 256x256x64 outweighs the extra work-groups
-    int nchunk = (512 + tiles - 1) / tiles;
-    const int maxch = g.nz / 8 > 1 ? g.nz / 8 : 1;
-    nchunk = nchunk > maxch ? maxch : nchunk;
-    if (m.tend_kc > 0) nchunk = (g.nz + m.tend_kc - 1) / m.tend_kc;
-    a.kc = (g.nz + nchunk - 1) / nchunk;
+    a.kc = m.tend_kc > 0 ? m.tend_kc : tendency_levels(tiles, g.nz);
     a.nchunk = (g.nz + a.kc - 1) / a.kc;
     a.nblocks = tiles * a.nchunk;
     hipLaunchKernelGGL(k_tendency_lds<T>, dim3((unsigned)a.nblocks), dim3(TTHR), 0, m.stream, m.c, a);
