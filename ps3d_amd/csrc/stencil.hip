@@ -125,15 +125,32 @@ __global__ __launch_bounds__(BX * BY) void k_tendency(StepConsts c, const double
 
 // ---------------------------------------------------------------------------
 // the same tendencies, LDS-tiled: a work-group owns a TTX x TTY column tile
-// and marches up a chunk of levels with planes k-1, k, k+1 of u, v, w, b
-// (tile plus a one-point apron) in an LDS ring; the next plane is fetched
-// into registers while the current level is computed, so every value is
-// read from memory once per work-group.
+// and marches up a chunk of levels with the planes of u, v, w, b (tile plus a
+// one-point apron) of levels k and k + 1 in LDS and level k + 2 on its way.
+// What level k needs of level k - 1 is carried in registers: the fluxes
+// through its lower faces, which level k - 1 formed as its upper ones from
+// the same operands, and w.
+//
+// Bound: memory, at large grids (256x256x64: 280 MB in 53 us, 5.3 TB/s).
+// Planes come straight into LDS, as in fric_body, and what a level needs of
+// the one below is not recomputed: FP64 61 -> 53 us at 256x256x64, 2.36 ->
+// 2.01 ms at 1024x1024x128; mixed 60 -> 52 us.  The mixed form is built for
+// two work-groups per CU (at three, 80 registers, it spills: 100 us).
 // ---------------------------------------------------------------------------
 constexpr int TTX = TEND_TX, TTY = TEND_TY;
-constexpr int TPX = TTX + 2, TPY = TTY + 2;
 constexpr int TTHR = TTX * TTY;
-constexpr int TPER = (TPX * TPY + TTHR - 1) / TTHR;   // plane values per thread
+
+// planes in LDS: rows widened to whole 16-byte chunks, see FricPlane
+template <class T>
+struct TendPlane {
+    static constexpr int CH = 16 / (int)sizeof(T);
+    static constexpr int OX = 2;                            // columns before the tile
+    static constexpr int W = (OX + TTX + 1 + CH - 1) / CH * CH;
+    static constexpr int ROWS = TTY + 2;
+    static constexpr int N = W * ROWS, NCH = N / CH;
+    static_assert(NCH <= TTHR, "one chunk per lane");
+    static constexpr int WAVES = 4;                         // least per SIMD, for the register allocation
+};
 
 template <class T>
 struct TendArgs {
@@ -145,103 +162,144 @@ struct TendArgs {
     int kc, nchunk, tiles_x, tiles_y, nblocks;
 };
 
+// one 16-byte (or 4-byte) direct-to-LDS load per lane: global address per
+// lane, LDS address lds + lane * BYTES (lds uniform in the wavefront)
+template <int BYTES>
+__device__ __forceinline__ void load_to_lds(const void *g, void *lds)
+{
+    const auto *gp = (const __attribute__((address_space(1))) void *)g;
+    auto *lp = (__attribute__((address_space(3))) void *)lds;
+    if constexpr (BYTES == 16) __builtin_amdgcn_global_load_lds(gp, lp, 16, 0, 0);
+    else __builtin_amdgcn_global_load_lds(gp, lp, 4, 0, 0);
+}
+
+// element o of the level that starts at p (uniform in the wavefront): the
+// offset within a level fits 32 bits, so that the address takes one vector
+// register and no 64-bit arithmetic.  (The empty statement keeps the
+// compiler from widening the offset once, outside the loop over levels, into
+// two registers that it then holds through the loop.)
+template <class T>
+__device__ __forceinline__ T &at(T *p, unsigned o)
+{
+    using B = std::conditional_t<std::is_const<T>::value, const char, char>;
+    asm volatile("" : "+v"(o));
+    return *reinterpret_cast<T *>(reinterpret_cast<B *>(p) + o * (unsigned)sizeof(T));
+}
+
 // The flux-form advection terms at interior point (i, j, k) of level k,
 // advection.f90:2-184: F(f, dk, dj, di) is field f (0..3: u, v, w, b) at
-// (i+di, j+dj, k+dk).  Each returns -Ro * (flux divergence) (times dsqr for
-// w), the expressions and their association those of the reference, so
-// every kernel that evaluates them through these helpers gets the same bits.
+// (i+di, j+dj, k+dk), dk = 0 or 1; ft is the flux through the point's lower
+// face and becomes that through its upper face.  Each returns -Ro * (flux
+// divergence) (times dsqr for w), the expressions and their association
+// those of the reference, so every kernel that evaluates them through these
+// helpers gets the same bits.  The flux functions are those of flux_top at
+// level k (0 <= k <= nz).
 template <class T, class A>
-__device__ __forceinline__ T adv_b(const StepConsts &c, int k, A F)
+__device__ __forceinline__ T flux_top_b(const StepConsts &c, int k, A F)
 {
-    const bool lid = c.lid != 0;
-    const bool top0 = lid && (k >= c.nz);
-    const bool bot0 = lid && (k - 1 <= 0);
-    const T h = T(0.5), zero = T(0), Ro = (T)c.Ro;
+    if (c.lid != 0 && (k <= 0 || k >= c.nz)) return T(0);
+    return T(0.5) * (F(3, 0, 0, 0) + F(3, 1, 0, 0)) * F(2, 0, 0, 0);
+}
+
+template <class T, class A>
+__device__ __forceinline__ T flux_top_u(const StepConsts &c, int k, A F)
+{
+    if (c.lid != 0 && (k <= 0 || k >= c.nz)) return T(0);
+    return T(0.25) * (F(0, 1, 0, 0) + F(0, 0, 0, 0)) * (F(2, 0, 0, 0) + F(2, 0, 0, 1));
+}
+
+template <class T, class A>
+__device__ __forceinline__ T flux_top_v(const StepConsts &c, int k, A F)
+{
+    if (c.lid != 0 && (k <= 0 || k >= c.nz)) return T(0);
+    return T(0.25) * (F(1, 1, 0, 0) + F(1, 0, 0, 0)) * (F(2, 0, 0, 0) + F(2, 0, 1, 0));
+}
+
+template <class T, class A>
+__device__ __forceinline__ T flux_top_w(const StepConsts &c, int k, A F)
+{
+    if (c.lid != 0 && (k <= 0 || k >= c.nz - 1)) return T(0);
+    return T(0.25) * (F(2, 1, 0, 0) + F(2, 0, 0, 0)) * (F(2, 0, 0, 0) + F(2, 1, 0, 0));
+}
+
+template <class T, class A>
+__device__ __forceinline__ T adv_b(const StepConsts &c, int k, T &ft, A F)
+{
+    const T h = T(0.5), Ro = (T)c.Ro;
     const T fe1 = h * (F(3, 0, 0, 0) + F(3, 0, 0, 1)) * F(0, 0, 0, 0);
     const T fe0 = h * (F(3, 0, 0, -1) + F(3, 0, 0, 0)) * F(0, 0, 0, -1);
     const T fn1 = h * (F(3, 0, 0, 0) + F(3, 0, 1, 0)) * F(1, 0, 0, 0);
     const T fn0 = h * (F(3, 0, -1, 0) + F(3, 0, 0, 0)) * F(1, 0, -1, 0);
-    const T ft1 = top0 ? zero : h * (F(3, 0, 0, 0) + F(3, 1, 0, 0)) * F(2, 0, 0, 0);
-    const T ft0 = bot0 ? zero : h * (F(3, -1, 0, 0) + F(3, 0, 0, 0)) * F(2, -1, 0, 0);
+    const T ft0 = ft;
+    ft = flux_top_b<T>(c, k, F);
     return -(Ro * (sdiv<T>(fe1 - fe0, c.dx, c.rdx) + sdiv<T>(fn1 - fn0, c.dy, c.rdy) +
-                   sdiv<T>(ft1 - ft0, c.dz, c.rdz)));
+                   sdiv<T>(ft - ft0, c.dz, c.rdz)));
 }
 
 template <class T, class A>
-__device__ __forceinline__ T adv_u(const StepConsts &c, int k, A F)
+__device__ __forceinline__ T adv_u(const StepConsts &c, int k, T &ft, A F)
 {
-    const bool lid = c.lid != 0;
-    const bool top0 = lid && (k >= c.nz);
-    const bool bot0 = lid && (k - 1 <= 0);
-    const T q4 = T(0.25), zero = T(0), Ro = (T)c.Ro;
+    const T q4 = T(0.25), Ro = (T)c.Ro;
     const T fe1 = q4 * (F(0, 0, 0, 0) + F(0, 0, 0, 1)) * (F(0, 0, 0, 1) + F(0, 0, 0, 0));
     const T fe0 = q4 * (F(0, 0, 0, -1) + F(0, 0, 0, 0)) * (F(0, 0, 0, 0) + F(0, 0, 0, -1));
     const T fn1 = q4 * (F(0, 0, 0, 0) + F(0, 0, 1, 0)) * (F(1, 0, 0, 1) + F(1, 0, 0, 0));
     const T fn0 = q4 * (F(0, 0, -1, 0) + F(0, 0, 0, 0)) * (F(1, 0, -1, 1) + F(1, 0, -1, 0));
-    const T ft1 = top0 ? zero : q4 * (F(0, 1, 0, 0) + F(0, 0, 0, 0)) * (F(2, 0, 0, 0) + F(2, 0, 0, 1));
-    const T ft0 = bot0 ? zero : q4 * (F(0, 0, 0, 0) + F(0, -1, 0, 0)) * (F(2, -1, 0, 0) + F(2, -1, 0, 1));
+    const T ft0 = ft;
+    ft = flux_top_u<T>(c, k, F);
     return -(Ro * (sdiv<T>(fe1 - fe0, c.dx, c.rdx) + sdiv<T>(fn1 - fn0, c.dy, c.rdy) +
-                   sdiv<T>(ft1 - ft0, c.dz, c.rdz)));
+                   sdiv<T>(ft - ft0, c.dz, c.rdz)));
 }
 
 template <class T, class A>
-__device__ __forceinline__ T adv_v(const StepConsts &c, int k, A F)
+__device__ __forceinline__ T adv_v(const StepConsts &c, int k, T &ft, A F)
 {
-    const bool lid = c.lid != 0;
-    const bool top0 = lid && (k >= c.nz);
-    const bool bot0 = lid && (k - 1 <= 0);
-    const T q4 = T(0.25), zero = T(0), Ro = (T)c.Ro;
+    const T q4 = T(0.25), Ro = (T)c.Ro;
     const T fe1 = q4 * (F(1, 0, 0, 0) + F(1, 0, 0, 1)) * (F(0, 0, 1, 0) + F(0, 0, 0, 0));
     const T fe0 = q4 * (F(1, 0, 0, -1) + F(1, 0, 0, 0)) * (F(0, 0, 1, -1) + F(0, 0, 0, -1));
     const T fn1 = q4 * (F(1, 0, 0, 0) + F(1, 0, 1, 0)) * (F(1, 0, 1, 0) + F(1, 0, 0, 0));
     const T fn0 = q4 * (F(1, 0, -1, 0) + F(1, 0, 0, 0)) * (F(1, 0, 0, 0) + F(1, 0, -1, 0));
-    const T ft1 = top0 ? zero : q4 * (F(1, 1, 0, 0) + F(1, 0, 0, 0)) * (F(2, 0, 0, 0) + F(2, 0, 1, 0));
-    const T ft0 = bot0 ? zero : q4 * (F(1, 0, 0, 0) + F(1, -1, 0, 0)) * (F(2, -1, 0, 0) + F(2, -1, 1, 0));
+    const T ft0 = ft;
+    ft = flux_top_v<T>(c, k, F);
     return -(Ro * (sdiv<T>(fe1 - fe0, c.dx, c.rdx) + sdiv<T>(fn1 - fn0, c.dy, c.rdy) +
-                   sdiv<T>(ft1 - ft0, c.dz, c.rdz)));
+                   sdiv<T>(ft - ft0, c.dz, c.rdz)));
 }
 
 template <class T, class A>
-__device__ __forceinline__ T adv_w(const StepConsts &c, int k, A F)
+__device__ __forceinline__ T adv_w(const StepConsts &c, int k, T &ft, A F)
 {
-    const bool lid = c.lid != 0;
-    const bool bot0 = lid && (k - 1 <= 0);
-    const bool top0w = lid && (k >= c.nz - 1);
-    const T q4 = T(0.25), zero = T(0), Ro = (T)c.Ro;
+    const T q4 = T(0.25), Ro = (T)c.Ro;
     const T fe1 = q4 * (F(2, 0, 0, 0) + F(2, 0, 0, 1)) * (F(0, 0, 0, 0) + F(0, 1, 0, 0));
     const T fe0 = q4 * (F(2, 0, 0, -1) + F(2, 0, 0, 0)) * (F(0, 0, 0, -1) + F(0, 1, 0, -1));
     const T fn1 = q4 * (F(2, 0, 0, 0) + F(2, 0, 1, 0)) * (F(1, 0, 0, 0) + F(1, 1, 0, 0));
     const T fn0 = q4 * (F(2, 0, -1, 0) + F(2, 0, 0, 0)) * (F(1, 0, -1, 0) + F(1, 1, -1, 0));
-    const T ft1 = top0w ? zero : q4 * (F(2, 1, 0, 0) + F(2, 0, 0, 0)) * (F(2, 0, 0, 0) + F(2, 1, 0, 0));
-    const T ft0 = (bot0 || (lid && k - 1 >= c.nz - 1))
-                      ? zero
-                      : q4 * (F(2, 0, 0, 0) + F(2, -1, 0, 0)) * (F(2, -1, 0, 0) + F(2, 0, 0, 0));
+    const T ft0 = ft;
+    ft = flux_top_w<T>(c, k, F);
     return -(((T)c.dsqr * Ro) * (sdiv<T>(fe1 - fe0, c.dx, c.rdx) + sdiv<T>(fn1 - fn0, c.dy, c.rdy) +
-                                 sdiv<T>(ft1 - ft0, c.dz, c.rdz)));
+                                 sdiv<T>(ft - ft0, c.dz, c.rdz)));
 }
 
 // The FP64 tendencies of integrate.f90:12-54 at interior point (i, j, k):
 // advection (when enable_nonlinear), then the inline terms -- N0^2 w for b,
 // Coriolis for u and v, buoyancy and the lid for w -- as the reference adds
-// them.  F as for adv_b.
+// them.  F and ft as for adv_b; wm is w(k - 1).
 template <int FLD, class A>
-__device__ __forceinline__ double tendency_fp64(const StepConsts &c, int k, A F)
+__device__ __forceinline__ double tendency_fp64(const StepConsts &c, int k, double &ft, double wm, A F)
 {
     const double h = 0.5, q4 = 0.25;
     double t = 0.0;
     if constexpr (FLD == 0) {
-        if (c.nonlinear) t = adv_u<double>(c, k, F);
+        if (c.nonlinear) t = adv_u<double>(c, k, ft, F);
         t = t + (F(1, 0, 0, 0) + F(1, 0, -1, 0) + F(1, 0, 0, 1) + F(1, 0, -1, 1)) * q4 * c.f0;
     } else if constexpr (FLD == 1) {
-        if (c.nonlinear) t = adv_v<double>(c, k, F);
+        if (c.nonlinear) t = adv_v<double>(c, k, ft, F);
         t = t - (F(0, 0, 0, -1) + F(0, 0, 0, 0) + F(0, 0, 1, -1) + F(0, 0, 1, 0)) * q4 * c.f0;
     } else if constexpr (FLD == 2) {
-        if (c.nonlinear) t = adv_w<double>(c, k, F);
+        if (c.nonlinear) t = adv_w<double>(c, k, ft, F);
         t = t + h * (F(3, 0, 0, 0) + F(3, 1, 0, 0));
         if (c.lid != 0 && k >= c.nz) t = 0.0;
     } else {
-        if (c.nonlinear) t = adv_b<double>(c, k, F);
-        t = t - h * (F(2, 0, 0, 0) + F(2, -1, 0, 0)) * (c.N0 * c.N0);
+        if (c.nonlinear) t = adv_b<double>(c, k, ft, F);
+        t = t - h * (F(2, 0, 0, 0) + wm) * (c.N0 * c.N0);
     }
     return t;
 }
@@ -251,142 +309,174 @@ __device__ __forceinline__ double tendency_fp64(const StepConsts &c, int k, A F)
 template <class T>
 __device__ __forceinline__ void tendency_body(const StepConsts &c, const TendArgs<T> &a, int bid)
 {
-    __shared__ T sp[4][3][TPY][TPX];
+    constexpr bool MIXED = std::is_same<T, float>::value;
+    using PL = TendPlane<T>;
+    constexpr int W = PL::W, OX = PL::OX, CH = PL::CH;
+    // three arrays, not one: see fric_body
+    __shared__ __attribute__((aligned(16))) T pl0[4 * PL::N], pl1[4 * PL::N], pl2[4 * PL::N];
     // tiles fastest: the work-groups resident on an XCD at once hold many
     // rows of tiles of the same chunk, which march through the same levels
     // together, so the apron rows a tile shares with its y-neighbours are
     // read from HBM once and then found in L2
     const int ntile = a.tiles_x * a.tiles_y;
-    const int tile = bid % ntile;
-    const int ch = bid / ntile;
-    const int i0 = (tile % a.tiles_x) * TTX + 1;
-    const int j0 = (tile / a.tiles_x) * TTY + 1;
+    const int tile = __builtin_amdgcn_readfirstlane(bid % ntile);   // (divisions run on the vector unit)
+    const int ch = __builtin_amdgcn_readfirstlane(bid / ntile);
+    const int i0 = __builtin_amdgcn_readfirstlane(tile % a.tiles_x) * TTX + 1;
+    const int j0 = __builtin_amdgcn_readfirstlane(tile / a.tiles_x) * TTY + 1;
     const int kb = 1 + ch * a.kc;
     const int ke = min(c.nz, kb + a.kc - 1);
     const int t = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int nx = c.nx, ny = c.ny, nz = c.nz;
-    const T *fld[4] = {a.u, a.v, a.w, a.b};
 
-    T pre[4][TPER];
-    auto fetch = [&](int k) {
-#pragma unroll
-        for (int s = 0; s < TPER; ++s) {
-            const int q = t + s * TTHR;
-            const int rx = q % TPX, ry = q / TPX;
-            const int ii = i0 - 1 + rx, jj = j0 - 1 + ry;
-            const bool ok = q < TPX * TPY && ii <= nx + 2 && jj <= ny + 2;
-            const int64_t o = idx(c, ii, jj, k);
-#pragma unroll
-            for (int f = 0; f < 4; ++f) pre[f][s] = ok ? fld[f][o] : T(0);
-        }
+    // loads of a plane, clamped as in fric_body
+    const bool chunks = sizeof(T) == 8 || c.X % CH == 0;
+    const int last = (int)c.X - (chunks ? CH : 1);
+    auto src = [&](int q) {   // element q of the plane, from the level's start
+        const int jj = min(j0 - 1 + q / W, ny + 2);
+        return (unsigned)min(i0 - OX + 1 + q % W, last) + (unsigned)c.X * (unsigned)(jj + 1);
     };
-    auto store = [&](int k) {
-        const int sl = (k - kb + 1) % 3;
+    const unsigned mysrc = src(t < PL::NCH ? t * CH : 0);
+    auto fetch = [&](T *dst, int k) {
+        const int64_t lk = c.XY * (int64_t)(k + 1);
+        const T *fld[4] = {a.u + lk, a.v + lk, a.w + lk, a.b + lk};
+        if (chunks) {
+            if (t < PL::NCH) {
 #pragma unroll
-        for (int s = 0; s < TPER; ++s) {
-            const int q = t + s * TTHR;
-            if (q < TPX * TPY) {
-                const int rx = q % TPX, ry = q / TPX;
+                for (int f = 0; f < 4; ++f) load_to_lds<16>(&at(fld[f], mysrc), dst + f * PL::N + wave * 64 * CH);
+            }
+        } else {
+            for (int s = 0; s * TTHR < PL::N; ++s) {
+                const int q = t + s * TTHR;
+                if (q < PL::N) {
+                    const unsigned o = src(q);
 #pragma unroll
-                for (int f = 0; f < 4; ++f) sp[f][sl][ry][rx] = pre[f][s];
+                    for (int f = 0; f < 4; ++f) load_to_lds<4>(&at(fld[f], o), dst + f * PL::N + s * TTHR + wave * 64);
+                }
             }
         }
     };
 
-    fetch(kb - 1);
-    store(kb - 1);
-    fetch(kb);
-    store(kb);
-    fetch(kb + 1);
     const int px = t % TTX, py = t / TTX;
     const int i = i0 + px, j = j0 + py;
-    const int rx = px + 1, ry = py + 1;
+    const bool mine = i <= nx && j <= ny;
+    const int q0 = (py + 1) * W + px + OX;   // the lane's point in a plane
     const bool lid = c.lid != 0;
     const T h = T(0.5), zero = T(0);
-    constexpr bool MIXED = std::is_same<T, float>::value;
-    for (int k = kb; k <= ke; ++k) {
-        store(k + 1);
-        if (k + 2 <= nz + 2 && k + 1 <= ke) fetch(k + 2);
-        // mixed form: the lo parts and the reference pressure this point
-        // needs, issued before the barrier
+    // the lane's point in memory, from the level's start; mixed form: the
+    // points before and after it along x (om, op) and the steps to the rows
+    // before and after it (jm, jp) at their periodic images inside the
+    // domain, where the lo parts are current (the kernels keep only the hi
+    // parts' halos so; under a lid b's level nz + 1 is not used)
+    const unsigned o2 = (unsigned)(i + 1) + (unsigned)c.X * (unsigned)(j + 1);
+    const unsigned om = o2 + (i == 1 ? (unsigned)(nx - 1) : ~0u), op = o2 - (i == nx ? (unsigned)(nx - 1) : ~0u);
+    const unsigned jm = j == 1 ? (unsigned)c.X * (unsigned)(ny - 1) : -(unsigned)c.X;
+    const unsigned jp = j == ny ? -((unsigned)c.X * (unsigned)(ny - 1)) : (unsigned)c.X;
+
+    fetch(pl0, kb - 1);
+    fetch(pl1, kb);
+    fetch(pl2, kb + 1);
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+    __syncthreads();
+    // carried upward: the fluxes through the lower faces, and w(k - 1)
+    T ftu = zero, ftv = zero, ftw = zero, ftb = zero;
+    {
+        auto F = [&](int f, int dk, int dj, int di) -> T { return (dk ? pl1 : pl0)[f * PL::N + q0 + dj * W + di]; };
+        ftu = flux_top_u<T>(c, kb - 1, F);
+        ftv = flux_top_v<T>(c, kb - 1, F);
+        ftw = flux_top_w<T>(c, kb - 1, F);
+        ftb = flux_top_b<T>(c, kb - 1, F);
+    }
+    T wm = pl0[2 * PL::N + q0];
+
+    // level k: the planes of levels k and k + 1 in sc and sp, those of level
+    // k + 2 fetched into sn meanwhile
+    auto level = [&](int k, const T *sc, const T *sp, T *sn) {
+        __syncthreads();
+        if (k + 1 <= ke) fetch(sn, k + 2);
+        // mixed form: the lo parts and the reference pressure this point needs
         float lu[4] = {}, lv[4] = {}, lb[2] = {};
         double pp[4] = {};
+        const int64_t lk = c.XY * (int64_t)(k + 1);
         if constexpr (MIXED) {
-            if (i <= nx && j <= ny) {
-                const int64_t o = idx(c, i, j, k);
-                const int64_t X = c.X, XY = c.XY;
-                // the lo parts at the neighbours' periodic partners inside
-                // the domain (the kernels keep only the hi parts' halos
-                // current; under a lid b's level nz + 1 is not used)
-                const int im = i == 1 ? nx : i - 1, ip = i == nx ? 1 : i + 1;
-                const int jm = j == 1 ? ny : j - 1, jp = j == ny ? 1 : j + 1;
-                const int kp = k == nz ? 1 : k + 1;
-                lu[0] = a.ul[idx(c, im, j, k)]; lu[1] = a.ul[o]; lu[2] = a.ul[idx(c, im, jp, k)];
-                lu[3] = a.ul[idx(c, i, jp, k)];
-                lv[0] = a.vl[o]; lv[1] = a.vl[idx(c, i, jm, k)]; lv[2] = a.vl[idx(c, ip, j, k)];
-                lv[3] = a.vl[idx(c, ip, jm, k)];
-                lb[0] = a.bl[o]; lb[1] = a.bl[idx(c, i, j, kp)];
+            if (mine) {
+                const float *ul = a.ul + lk, *vl = a.vl + lk;
+                lu[0] = at(ul, om); lu[1] = at(ul, o2); lu[2] = at(ul, om + jp); lu[3] = at(ul, o2 + jp);
+                lv[0] = at(vl, o2); lv[1] = at(vl, o2 + jm); lv[2] = at(vl, op); lv[3] = at(vl, op + jm);
+                lb[0] = at(a.bl + lk, o2);
+                lb[1] = at(a.bl + c.XY * (int64_t)(k == nz ? 2 : k + 2), o2);
                 if (a.pint) {
-                    pp[0] = a.pint[o]; pp[1] = a.pint[o + 1]; pp[2] = a.pint[o + X]; pp[3] = a.pint[o + XY];
+                    const double *pi = a.pint + lk;
+                    pp[0] = at(pi, o2); pp[1] = at(pi, o2 + 1); pp[2] = at(pi, o2 + (unsigned)c.X);
+                    pp[3] = at(pi + c.XY, o2);
                 }
             }
         }
-        __syncthreads();
-        const int sm = (k - kb) % 3, sc = (k - kb + 1) % 3, sx = (k - kb + 2) % 3;
-        if (i <= nx && j <= ny) {
-            // value of field f at (i+di, j+dj, k+dk)
-            auto F = [&](int f, int dk, int dj, int di) -> T {
-                const int sl = dk < 0 ? sm : (dk > 0 ? sx : sc);
-                return sp[f][sl][ry + dj][rx + di];
-            };
-            auto U = [&](int dk, int dj, int di) { return F(0, dk, dj, di); };
-            auto V = [&](int dk, int dj, int di) { return F(1, dk, dj, di); };
-            auto W = [&](int dk, int dj, int di) { return F(2, dk, dj, di); };
-            auto B = [&](int dk, int dj, int di) { return F(3, dk, dj, di); };
-            const int64_t o = idx(c, i, j, k);
-            if constexpr (!MIXED) {
-                a.db[o] = tendency_fp64<3>(c, k, F);
-                a.du[o] = tendency_fp64<0>(c, k, F);
-                a.dv[o] = tendency_fp64<1>(c, k, F);
-                a.dw[o] = tendency_fp64<2>(c, k, F);
-            } else {
-                T adv = zero, au = zero, av = zero, aw = zero;
-                if (c.nonlinear) {
-                    adv = adv_b<T>(c, k, F);
-                    au = adv_u<T>(c, k, F);
-                    av = adv_v<T>(c, k, F);
-                    aw = adv_w<T>(c, k, F);
-                }
-                adv = adv - h * (W(0, 0, 0) + W(-1, 0, 0)) * (T)(c.N0 * c.N0);
-                a.db[o] = adv;
-                // mixed form: the Coriolis and buoyancy terms, which the
-                // pressure gradient nearly balances, and that gradient in FP64
-                // from (hi, lo); the slots keep tendency - grad(pint)
-                auto u64 = [&](int dj, int di, int q) { return (double)U(0, dj, di) + (double)lu[q]; };
-                auto v64 = [&](int dj, int di, int q) { return (double)V(0, dj, di) + (double)lv[q]; };
-                const double cu = (v64(0, 0, 0) + v64(-1, 0, 1) + v64(0, 1, 2) + v64(-1, 1, 3)) * 0.25 * c.f0;
-                const double cv = (u64(0, -1, 0) + u64(0, 0, 1) + u64(1, -1, 2) + u64(1, 0, 3)) * 0.25 * c.f0;
-                const double bb = 0.5 * (((double)B(0, 0, 0) + (double)lb[0]) + ((double)B(1, 0, 0) + (double)lb[1]));
-                double gx = 0.0, gy = 0.0, gz = 0.0;
-                if (a.pint) {
-                    gx = (pp[1] - pp[0]) * c.rdx;
-                    gy = (pp[2] - pp[0]) * c.rdy;
-                    gz = (pp[3] - pp[0]) * c.rdz;
-                }
-                const double su = ((double)au + cu) - gx;
-                const double sv = ((double)av - cv) - gy;
-                const double sw = (lid && k >= nz) ? 0.0 : ((double)aw + bb) - gz;
-                a.du[o] = (float)su;
-                a.dv[o] = (float)sv;
-                a.dw[o] = (float)sw;
+        // value of field f at (i+di, j+dj, k+dk)
+        auto F = [&](int f, int dk, int dj, int di) -> T { return (dk ? sp : sc)[f * PL::N + q0 + dj * W + di]; };
+        if constexpr (!MIXED) {
+            const double rb = tendency_fp64<3>(c, k, ftb, wm, F);
+            const double ru = tendency_fp64<0>(c, k, ftu, wm, F);
+            const double rv = tendency_fp64<1>(c, k, ftv, wm, F);
+            const double rw = tendency_fp64<2>(c, k, ftw, wm, F);
+            wm = F(2, 0, 0, 0);
+            // the next planes have arrived before this level's stores begin,
+            // so the wait is never for them
+            __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+            if (mine) {
+                at(a.db + lk, o2) = rb;
+                at(a.du + lk, o2) = ru;
+                at(a.dv + lk, o2) = rv;
+                at(a.dw + lk, o2) = rw;
+            }
+        } else {
+            T adv = zero, au = zero, av = zero, aw = zero;
+            if (c.nonlinear) {
+                adv = adv_b<T>(c, k, ftb, F);
+                au = adv_u<T>(c, k, ftu, F);
+                av = adv_v<T>(c, k, ftv, F);
+                aw = adv_w<T>(c, k, ftw, F);
+            }
+            adv = adv - h * (F(2, 0, 0, 0) + wm) * (T)(c.N0 * c.N0);
+            wm = F(2, 0, 0, 0);
+            // mixed form: the Coriolis and buoyancy terms, which the
+            // pressure gradient nearly balances, and that gradient in FP64
+            // from (hi, lo); the slots keep tendency - grad(pint)
+            auto u64 = [&](int dj, int di, int q) { return (double)F(0, 0, dj, di) + (double)lu[q]; };
+            auto v64 = [&](int dj, int di, int q) { return (double)F(1, 0, dj, di) + (double)lv[q]; };
+            const double cu = (v64(0, 0, 0) + v64(-1, 0, 1) + v64(0, 1, 2) + v64(-1, 1, 3)) * 0.25 * c.f0;
+            const double cv = (u64(0, -1, 0) + u64(0, 0, 1) + u64(1, -1, 2) + u64(1, 0, 3)) * 0.25 * c.f0;
+            const double bb = 0.5 * (((double)F(3, 0, 0, 0) + (double)lb[0]) + ((double)F(3, 1, 0, 0) + (double)lb[1]));
+            double gx = 0.0, gy = 0.0, gz = 0.0;
+            if (a.pint) {
+                gx = (pp[1] - pp[0]) * c.rdx;
+                gy = (pp[2] - pp[0]) * c.rdy;
+                gz = (pp[3] - pp[0]) * c.rdz;
+            }
+            const double su = ((double)au + cu) - gx;
+            const double sv = ((double)av - cv) - gy;
+            const double sw = (lid && k >= nz) ? 0.0 : ((double)aw + bb) - gz;
+            __builtin_amdgcn_s_waitcnt(0x0f70);   // as above
+            if (mine) {
+                at(a.db + lk, o2) = adv;
+                at(a.du + lk, o2) = (float)su;
+                at(a.dv + lk, o2) = (float)sv;
+                at(a.dw + lk, o2) = (float)sw;
             }
         }
-        __syncthreads();
+    };
+    for (int k = kb;;) {
+        level(k, pl1, pl2, pl0);
+        if (++k > ke) break;
+        level(k, pl2, pl0, pl1);
+        if (++k > ke) break;
+        level(k, pl0, pl1, pl2);
+        if (++k > ke) break;
     }
 }
 
 template <class T>
-__global__ __launch_bounds__(TTHR) void k_tendency_lds(StepConsts c, TendArgs<T> a)
+__global__ __launch_bounds__(TTHR, TendPlane<T>::WAVES) void k_tendency_lds(StepConsts c, TendArgs<T> a)
 {
     tendency_body<T>(c, a, xcd_remap((int)blockIdx.x, a.nblocks));
 }
@@ -748,7 +838,7 @@ struct FricPlane {
     static constexpr int ROWS = FTY + 6;
     static constexpr int N = W * ROWS, NCH = N / CH;
     static_assert(NCH <= FTHREADS, "one chunk per lane");
-    static constexpr int WAVES = sizeof(T) == 8 ? 1 : 6;    // least per SIMD, for the register allocation
+    static constexpr int WAVES = sizeof(T) == 8 ? 1 : 8;    // least per SIMD, for the register allocation
 };
 
 template <class T>
@@ -784,18 +874,7 @@ struct FricArgs {
 template <class T>
 __device__ __forceinline__ int fric_field(const FricArgs<T> &a, int bid)
 {
-    return bid / (a.tiles_x * a.tiles_y) / a.nchunk;
-}
-
-// one 16-byte (or 4-byte) direct-to-LDS load per lane: global address per
-// lane, LDS address lds + lane * BYTES (lds uniform in the wavefront)
-template <int BYTES>
-__device__ __forceinline__ void load_to_lds(const void *g, void *lds)
-{
-    const auto *gp = (const __attribute__((address_space(1))) void *)g;
-    auto *lp = (__attribute__((address_space(3))) void *)lds;
-    if constexpr (BYTES == 16) __builtin_amdgcn_global_load_lds(gp, lp, 16, 0, 0);
-    else __builtin_amdgcn_global_load_lds(gp, lp, 4, 0, 0);
+    return __builtin_amdgcn_readfirstlane(bid / (a.tiles_x * a.tiles_y) / a.nchunk);
 }
 
 template <class T>
@@ -804,6 +883,8 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
     constexpr bool MIXED = std::is_same<T, float>::value;
     using PL = FricPlane<T>;
     constexpr int W = PL::W, OX = PL::OX, CH = PL::CH;
+    constexpr int OFF = 8;   // the first tile's planes begin OX - 2 elements before a row: offsets stay positive
+    static_assert(OFF % CH == 0 && OFF >= OX, "whole chunks");
     // f0 of three levels.  Three arrays, not one: the compiler then knows
     // that reads of one need not wait for loads into another.
     __shared__ __attribute__((aligned(16))) T pl0[PL::N], pl1[PL::N], pl2[PL::N];
@@ -811,11 +892,10 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
     __shared__ T d2p[FTY + 2][FTX + 2];   // biharmonic_h's del2 on the tile + 1
     __shared__ T hinc[MIXED ? FTY : 1][MIXED ? FTX : 1];   // harmonic increment at tile points
     const int ntile = a.tiles_x * a.tiles_y;
-    const int tile = bid % ntile;
-    const int rest = bid / ntile;
-    const int ch = rest % a.nchunk;
-    const int i0 = (tile % a.tiles_x) * FTX + 1;   // x-adjacent tiles run together
-    const int j0 = (tile / a.tiles_x) * FTY + 1;
+    const int tile = __builtin_amdgcn_readfirstlane(bid % ntile);   // (divisions run on the vector unit)
+    const int ch = __builtin_amdgcn_readfirstlane(bid / ntile % a.nchunk);
+    const int i0 = __builtin_amdgcn_readfirstlane(tile % a.tiles_x) * FTX + 1;   // x-adjacent tiles run together
+    const int j0 = __builtin_amdgcn_readfirstlane(tile / a.tiles_x) * FTY + 1;
     const int kb = 1 + ch * a.kc;
     const int ke = min(c.nz, kb + a.kc - 1);
     const int t = threadIdx.x;
@@ -826,28 +906,31 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
     const T dt = (T)c.dt;
     const T zero = T(0);
 
-    // loads of a plane: rows past the array's are clamped, columns past a
-    // row's ends run into the rows beside (in the array: a level lies on
-    // either side); neither enters a stored value
+    // loads of a plane: rows and columns past the array's are clamped, columns
+    // before a row's start run into the row before (in the array: a level lies
+    // below); neither enters a stored value
     const bool chunks = sizeof(T) == 8 || c.X % CH == 0;   // rows start at 16-byte boundaries
-    auto src = [&](int q) {   // element q of the plane, from the level's start
+    const int last = (int)c.X - (chunks ? CH : 1);         // start of a row's last load
+    auto src = [&](int q) {   // element q of the plane, from OFF before the level's start
         const int jj = min(max(j0 - 3 + q / W, -1), ny + 2);
-        return (int64_t)(i0 - OX + 1 + q % W) + c.X * (int64_t)(jj + 1);
+        return (unsigned)(min(i0 - OX + 1 + q % W, last) + OFF) + (unsigned)c.X * (unsigned)(jj + 1);
     };
-    const T *mysrc = F.in + src(t < PL::NCH ? t * CH : 0);
+    const unsigned mysrc = src(t < PL::NCH ? t * CH : 0);
     auto fetch = [&](T *dst, int k) {
-        const int64_t lk = c.XY * (int64_t)(k + 1);
+        const T *lev = F.in + c.XY * (int64_t)(k + 1) - OFF;
         if (chunks) {
-            if (t < PL::NCH) load_to_lds<16>(mysrc + lk, dst + wave * 64 * CH);
+            if (t < PL::NCH) load_to_lds<16>(&at(lev, mysrc), dst + wave * 64 * CH);
         } else {
             for (int s = 0; s * FTHREADS < PL::N; ++s) {
                 const int q = t + s * FTHREADS;
-                if (q < PL::N) load_to_lds<4>(F.in + src(q) + lk, dst + s * FTHREADS + wave * 64);
+                if (q < PL::N) load_to_lds<4>(&at(lev, src(q)), dst + s * FTHREADS + wave * 64);
             }
         }
     };
     const int tpx = t % FTX, tpy = t / FTX;
     const bool mine = (i0 + tpx <= nx) && (j0 + tpy <= ny);
+    // the lane's point in memory, from the level's start
+    const unsigned o2 = (unsigned)(i0 + tpx + 1) + (unsigned)c.X * (unsigned)(j0 + tpy + 1);
 
     // the tendency slots (and lo part) of a level at the lane's point, read
     // once: streamed past the L2, which keeps the f0 planes that
@@ -859,18 +942,18 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
     auto load_pt = [&](int k) {
         Pt r{zero, zero, zero, zero, 0.f, 0.f, 0.f, 0.f};
         if (mine) {
-            const int64_t o = idx(c, i0 + tpx, j0 + tpy, k);
-            if (a.order >= 1) r.s0 = __builtin_nontemporal_load(F.t0 + o);
-            if (a.order >= 2) r.s1 = __builtin_nontemporal_load(F.t1 + o);
-            if (a.order >= 3) r.s2 = __builtin_nontemporal_load(F.t2 + o);
+            const int64_t lk = c.XY * (int64_t)(k + 1);
+            if (a.order >= 1) r.s0 = __builtin_nontemporal_load(&at(F.t0 + lk, o2));
+            if (a.order >= 2) r.s1 = __builtin_nontemporal_load(&at(F.t1 + lk, o2));
+            if (a.order >= 3) r.s2 = __builtin_nontemporal_load(&at(F.t2 + lk, o2));
             if constexpr (MIXED) {
-                r.lo0 = F.in_lo[o];
+                r.lo0 = at(F.in_lo + lk, o2);
                 if (F.gstride && a.d1) {
-                    r.q1o = a.d1[o];
-                    r.q1n = a.d1[o + F.gstride];
+                    r.q1o = at(a.d1 + lk, o2);
+                    r.q1n = at(a.d1 + (lk + F.gstride), o2);
                     if (a.d2) {
-                        r.q2o = a.d2[o];
-                        r.q2n = a.d2[o + F.gstride];
+                        r.q2o = at(a.d2 + lk, o2);
+                        r.q2n = at(a.d2 + (lk + F.gstride), o2);
                     }
                 }
             }
@@ -964,7 +1047,7 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
                 binc = dt * (sdiv<T>(fe1 - fe0, dx, rdx) + sdiv<T>(fn1 - fn0, dy, rdy));
                 f2 = f2 + binc;
             }
-            const int64_t o = idx(c, i, j, k);
+            const int64_t lk = c.XY * (int64_t)(k + 1);
             if constexpr (!MIXED) {
                 const double s = F.scale;
                 double val;
@@ -972,7 +1055,7 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
                 else if (a.order == 1) val = f2 + s * cur.s0;
                 else if (a.order == 2) val = f2 + s * (a.ca * cur.s0 - a.cb * cur.s1);
                 else val = f2 + s * (a.ca * cur.s0 + a.cb * cur.s1 + a.cc * cur.s2);
-                F.out[o] = val;
+                at(F.out + lk, o2) = val;
                 if (a.halo) write_images<double>(c, F.out, i, j, k, val, 0);
             } else {
                 const double s = F.scale;
@@ -996,8 +1079,8 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
                 }
                 const double x = base + ((zt ? 0.0 : (double)hinc[py][px]) + (double)binc + ab - gq);
                 const float hi = (float)x;
-                F.out[o] = hi;
-                F.out_lo[o] = (float)(x - (double)hi);
+                at(F.out + lk, o2) = hi;
+                at(F.out_lo + lk, o2) = (float)(x - (double)hi);
                 if (a.halo) write_images<float>(c, F.out, i, j, k, hi, 0);
             }
         }
@@ -1255,7 +1338,7 @@ inline dim3 full_grid(const Grid &g)
 // ---------------------------------------------------------------------------
 // batched ensemble stages: one launch over all members (see EnsMember)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(TTHR) void k_ens_tendency(const EnsMember *__restrict__ mem, EnsMap map,
+__global__ __launch_bounds__(TTHR, TendPlane<double>::WAVES) void k_ens_tendency(const EnsMember *__restrict__ mem, EnsMap map,
                                                         const EnsState *__restrict__ st)
 {
     const int g = xcd_remap((int)blockIdx.x, map.start[map.n]);
@@ -1549,7 +1632,7 @@ __global__ void k_ens_advance(EnsState *st)
 // ---- the same stages for members of the mixed form -------------------------
 // (the bodies and arguments of tendency_impl<float>, friction_ab_impl<float>
 // and k_project_f, with the member's buffers of the current parity)
-__global__ __launch_bounds__(TTHR) void k_ens_tendency_f(const EnsMember *__restrict__ mem, EnsMap map,
+__global__ __launch_bounds__(TTHR, TendPlane<float>::WAVES) void k_ens_tendency_f(const EnsMember *__restrict__ mem, EnsMap map,
                                                           const EnsState *__restrict__ st, int cold)
 {
     const int g = xcd_remap((int)blockIdx.x, map.start[map.n]);

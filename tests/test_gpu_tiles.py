@@ -1,0 +1,62 @@
+"""The tiled stencil kernels at the edges of their tiles and chunks.
+
+The tendency and friction kernels own 64 x 8 columns and march up chunks of
+levels whose planes go to LDS in 16-byte loads (4-byte ones where rows do not
+start at 16-byte boundaries: FP32 with nx % 4 == 2).  Sizes: the smallest
+grid, extents below, at and just past a tile, remainders of a chunk.  FP64
+follows the oracle bit for bit; the mixed form stays within the 1e-5 that its
+FP32 stencils are allowed elsewhere.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(2, 2, 2), (4, 4, 4), (6, 4, 5), (60, 16, 9), (64, 8, 3), (64, 10, 17), (72, 18, 6), (128, 6, 35)]
+
+
+def _pair(make, precision=None):
+    import oracle
+    from ps3d_amd.model import Model
+    prm, fields = make
+    gpu = Model(prm if precision is None else prm.replace(precision=precision))
+    orc = oracle.OracleModel(prm)
+    for n, a in fields.items():
+        gpu.f[n][...] = a
+        orc.f[n][...] = a
+    gpu.push()
+    return prm, gpu, orc
+
+
+@pytest.mark.parametrize("lid", [True, False])
+@pytest.mark.parametrize("size", SIZES)
+def test_fused_step_bitwise(size, lid):
+    from ps3d_amd import configs
+    nx, ny, nz = size
+    if not lid:
+        nz += nz % 2
+    print(f"steps {nx}x{ny}x{nz} lid={lid}", flush=True)
+    prm, gpu, orc = _pair(configs.random_state(nx, ny, nz, lid=lid, Avbi=0.0, Kvbi=0.0))
+    gpu.run(4)
+    orc.run(4)
+    gpu.pull()
+    for n in ("u", "v", "w", "b", "p"):
+        assert np.array_equal(gpu.f[n], orc.f[n]), n
+    gpu.close()
+    orc.close()
+
+
+@pytest.mark.parametrize("size", [(16, 8, 4), (30, 8, 5), (30, 30, 6), (64, 10, 17), (80, 16, 9)])
+def test_mixed_step(size):
+    from ps3d_amd import configs, diagnose
+    from ps3d_amd.params import PS3D_MIXED
+    print(f"mixed steps {size}", flush=True)
+    prm, gpu, orc = _pair(configs.jets(*size, seed=4), PS3D_MIXED)
+    gpu.run(4)
+    orc.run(4)
+    gpu.pull()
+    err = diagnose.compare(gpu.f, {n: orc.f[n] for n in ("u", "v", "w", "b", "p")}, prm)
+    for k in ("u", "v", "w", "b"):
+        assert err[k] <= 1e-5, (k, err[k])
+    gpu.close()
+    orc.close()
