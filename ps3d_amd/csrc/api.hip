@@ -285,9 +285,9 @@ void integrate(Model &m, int itt, int tau, int taum1, int taum2)
     }
     const bool forced = m.forcing || m.wm_on || background_on(m);
     launch_tendency(m, tau);
-    if (fused_friction_ok(m) && m.fuse_friction && !forced) {
+    if (fused_friction_ok(m) && !forced) {
         launch_friction_ab(m, itt, tau, taum1, taum2);
-    } else if (fused_friction_ok(m) && m.fuse_friction) {
+    } else if (fused_friction_ok(m)) {
         // set_forcing sees the post-friction state (integrate.f90:82)
         launch_friction_fused_only(m);
         if (!m.wm_on && !m.forcing) {
@@ -296,9 +296,11 @@ void integrate(Model &m, int itt, int tau, int taum1, int taum2)
             apply_forcing(m, itt, tau);
             launch_ab_exchange(m, itt, tau, taum1, taum2);
         }
+    } else if (!forced) {
+        launch_friction_block_ab(m, itt, tau, taum1, taum2);
     } else {
         launch_friction_block(m);
-        if (forced) apply_forcing(m, itt, tau);
+        apply_forcing(m, itt, tau);
         launch_ab_exchange(m, itt, tau, taum1, taum2);
     }
     pressure(m);
@@ -359,7 +361,7 @@ std::vector<uint64_t> graph_signature(const Model &m, const int32_t *st)
     h = fnv(h, &m.c, sizeof(m.c));
     h = fnv(h, &m.prm, sizeof(m.prm));
     const int opts[] = {m.tend_kc, m.fric_kc, m.thomas_cpw, (int)m.thomas_reg,
-                        (int)m.fuse_friction, (int)m.fuse_halo, m.fft_plan[0], m.fft_plan[1], m.fft_plan[2],
+                        (int)m.fuse_halo, m.fft_plan[0], m.fft_plan[1], m.fft_plan[2],
                         (int)m.bg_on, (int)m.bg_b_on, (int)m.bf_on[0], (int)m.bf_on[1], (int)m.bf_on[2],
                         (int)m.bf_on[3]};
     h = fnv(h, opts, sizeof(opts));

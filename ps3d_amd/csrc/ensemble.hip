@@ -21,7 +21,7 @@ using namespace ps3d;
 namespace {
 
 // S_PTS: 256 points per work-group over the H points of a member
-enum Stage { S_TEND, S_FRIC, S_R2C, S_COLS, S_THOMAS, S_ZSOLVE, S_PROJ, S_PTS, S_HCOPY, S_BGAB, S_NSTAGE };
+enum Stage { S_TEND, S_FRIC, S_R2C, S_COLS, S_THOMAS, S_ZSOLVE, S_PROJ, S_PTS, S_BGAB, S_NSTAGE };
 
 // tile shapes of the k-marching kernels (stencil.hip)
 constexpr int kTTX = TEND_TX, kTTY = TEND_TY, kFTX = FRIC_TX, kFTY = FRIC_TY;
@@ -145,14 +145,16 @@ void build_maps(ps3d_ensemble &E)
             int64_t nb = 0;
             switch (s) {
             case S_TEND: nb = (int64_t)e.tend_tx * e.tend_ty * e.tend_nchunk; break;
-            case S_FRIC: nb = (int64_t)e.fric_tx * e.fric_ty * e.fric_nchunk * 4; break;
+            case S_FRIC:   // forced: and the halo copies, four fields'
+                nb = (int64_t)e.fric_tx * e.fric_ty * e.fric_nchunk * 4;
+                if (e.forced) nb += 4 * cdiv(g.H - g.N, FRIC_HALO);
+                break;
             case S_R2C: nb = ens_r2c_blocks(e); break;
             case S_COLS: nb = ens_cols_blocks(e, g.ny, g.nz); break;
             case S_THOMAS: nb = lid ? cdiv((int64_t)g.nkx * g.ny, ens_thomas_cols(E.thomas_reg, E.thomas_split)) : 0; break;
             case S_ZSOLVE: nb = lid ? 0 : ens_cols_blocks(e, g.nz, g.ny); break;
             case S_PROJ: nb = (int64_t)cdiv(g.nx, 64) * cdiv(g.ny, 4) * g.nz; break;
             case S_PTS: nb = E.mixed ? cdiv(g.H, 256) : 0; break;
-            case S_HCOPY: nb = e.forced ? 4 * cdiv(g.H - g.N, 256) : 0; break;
             case S_BGAB: nb = e.forced ? (int64_t)cdiv(g.nx, 64) * cdiv(g.ny, 4) * g.nz : 0; break;
             }
             E.maps[s].start[i] = (int)acc;
@@ -252,9 +254,8 @@ void enqueue_step_mixed(ps3d_ensemble &E, bool refine)
     hipStream_t s = E.stream;
     ens_tendency_f(s, E.dev_tab, E.maps[S_TEND], E.dev_state, 0);
     ens_friction_ab_f(s, E.dev_tab, E.maps[S_FRIC], E.dev_state, 0);   // writes the halo images too
-    // forced members (their friction went to the third (hi, lo) buffers):
-    // the pre-friction hi halos, then forcing + Adams-Bashforth
-    ens_halo_copy(s, E.dev_tab, E.maps[S_HCOPY], E.dev_state, true);
+    // forced members (their friction went to the third (hi, lo) buffers, with
+    // the pre-friction hi halos): forcing + Adams-Bashforth
     ens_background_ab_f(s, E.dev_tab, E.maps[S_BGAB], E.dev_state);
     enqueue_solve_f(E, 1);
     ens_project_f(s, E.dev_tab, E.maps[S_PROJ], E.dev_state, 1);
@@ -276,9 +277,8 @@ void enqueue_step(ps3d_ensemble &E)
     hipStream_t s = E.stream;
     ens_tendency(s, E.dev_tab, E.maps[S_TEND], E.dev_state);
     ens_friction_ab(s, E.dev_tab, E.maps[S_FRIC], E.dev_state);   // writes the halo images too
-    // forced members (their friction went to the third buffers): the
-    // pre-friction halos, then set_forcing (integrate.f90:82) and AB
-    ens_halo_copy(s, E.dev_tab, E.maps[S_HCOPY], E.dev_state, false);
+    // forced members (their friction went to the third buffers, with the
+    // pre-friction halos): set_forcing (integrate.f90:82) and AB
     ens_background_ab(s, E.dev_tab, E.maps[S_BGAB], E.dev_state);
     ens_r2c(s, E.dev_tab, E.maps[S_R2C], E.dev_state, E.lds_x);
     ens_cols_y(s, E.dev_tab, E.maps[S_COLS], -1, E.ny_max, E.lds_y);

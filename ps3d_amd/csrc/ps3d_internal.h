@@ -70,6 +70,7 @@ constexpr int ONX = 2;   // halo width, main_module.f90:93
 #endif
 constexpr int TEND_TX = PS3D_TEND_TX, TEND_TY = PS3D_TEND_TY;
 constexpr int FRIC_TX = 64, FRIC_TY = PS3D_FRIC_TY;
+constexpr int FRIC_HALO = 4 * FRIC_TX * FRIC_TY;   // halo points that one work-group copies
 
 // Extents of one model.  Physical fields are (X, Y, Z) = (nx+4, ny+4, nz+4)
 // with Fortran index i in -1..nx+2 at offset i+1 (i fastest).
@@ -144,8 +145,10 @@ __device__ __forceinline__ int xcd_remap(int bid, int n)
 
 inline bool halo_images_ok(int nx, int ny, int nz) { return nx >= 4 && ny >= 4 && nz >= 4; }
 
-template <class T>
-__device__ __forceinline__ void write_images(const StepConsts &c, T *a, int i, int j, int k, T val, int neumann_z)
+// visit(o, kk): the halo points that are images of interior point (i, j, k),
+// by their offset in the array and their level
+template <class V>
+__device__ __forceinline__ void for_images(const StepConsts &c, int i, int j, int k, int neumann_z, V visit)
 {
     const int ox = i <= 2 ? c.nx : (i >= c.nx - 1 ? -c.nx : 0);
     const int oy = j <= 2 ? c.ny : (j >= c.ny - 1 ? -c.ny : 0);
@@ -153,25 +156,32 @@ __device__ __forceinline__ void write_images(const StepConsts &c, T *a, int i, i
     if (neumann_z) oz = k == 1 ? -1 : (k == c.nz ? 1 : 0);
     else oz = k <= 2 ? c.nz : (k >= c.nz - 1 ? -c.nz : 0);
     if ((ox | oy | oz) == 0) return;
-    T *p = a + (int64_t)(i + 1) + c.X * (int64_t)(j + 1) + c.XY * (int64_t)(k + 1);
+    const int64_t p = (int64_t)(i + 1) + c.X * (int64_t)(j + 1) + c.XY * (int64_t)(k + 1);
     const int64_t sx = ox, sy = (int64_t)oy * c.X;
-    if (ox) p[sx] = val;
+    if (ox) visit(p + sx, k);
     if (oy) {
-        p[sy] = val;
-        if (ox) p[sx + sy] = val;
+        visit(p + sy, k);
+        if (ox) visit(p + sx + sy, k);
     }
     if (oz) {
         const int nzi = neumann_z ? 2 : 1;   // Neumann: two copies, at distance 1 and 2
         for (int r = 1; r <= nzi; ++r) {
-            T *q = p + (int64_t)(oz * r) * c.XY;
-            q[0] = val;
-            if (ox) q[sx] = val;
+            const int64_t q = p + (int64_t)(oz * r) * c.XY;
+            const int kk = k + oz * r;
+            visit(q, kk);
+            if (ox) visit(q + sx, kk);
             if (oy) {
-                q[sy] = val;
-                if (ox) q[sx + sy] = val;
+                visit(q + sy, kk);
+                if (ox) visit(q + sx + sy, kk);
             }
         }
     }
+}
+
+template <class T>
+__device__ __forceinline__ void write_images(const StepConsts &c, T *a, int i, int j, int k, T val, int neumann_z)
+{
+    for_images(c, i, j, k, neumann_z, [&](int64_t o, int) { a[o] = val; });
 }
 
 // complex type of a real type
@@ -216,7 +226,6 @@ struct Model {
     // per-field "current buffer" during the friction block (0 = canonical)
     int cur[4] = {0, 0, 0, 0};
     // use the fused friction + Adams-Bashforth kernel where it applies
-    bool fuse_friction = true;
     // producers write the halo images of what they update (halo_images_ok)
     bool fuse_halo = false;
     // launch shapes (results do not depend on them; set by ps3d_tune):
@@ -294,6 +303,7 @@ void launch_tendency(Model &m, int tau);
 void launch_buoyancy_advection(Model &m, int tau);
 void launch_momentum_advection(Model &m, int tau);
 void launch_friction_block(Model &m);
+void launch_friction_block_ab(Model &m, int itt, int tau, int taum1, int taum2);
 void launch_mixing(Model &m, int op, int field, double hmix, double vmix, int zero_top);
 void launch_ab_exchange(Model &m, int itt, int tau, int taum1, int taum2);
 // the wavemaker on the current buffers: q += dt*(cs*re + sn*im), interior
@@ -468,7 +478,6 @@ void ens_friction_ab(hipStream_t s, const EnsMember *mem, const EnsMap &map, con
 void ens_project(hipStream_t s, const EnsMember *mem, const EnsMap &map, const EnsState *st);
 // forced FP64 members: pre-friction halos into the third buffers (4 fields x
 // halo points per member), then forcing + AB (interior points per member)
-void ens_halo_copy(hipStream_t s, const EnsMember *mem, const EnsMap &map, const EnsState *st, bool mixed);
 void ens_background_ab(hipStream_t s, const EnsMember *mem, const EnsMap &map, const EnsState *st);
 // mixed form: the forcing on the pre-friction state into slot tau (the cold
 // start's provisional step), and forcing + Adams-Bashforth from the third
@@ -504,7 +513,7 @@ void ens_thomas(hipStream_t s, const EnsMember *mem, const EnsMap &map, int nz_m
 // applies (0: dpr[0], the cold start's estimate; 1: the new increment
 // dpr[dp_cur + 1]; 2: the correction dpr[dp_cur + 2])
 void ens_tendency_f(hipStream_t s, const EnsMember *mem, const EnsMap &map, const EnsState *st, int cold);
-void ens_friction_ab_f(hipStream_t s, const EnsMember *mem, const EnsMap &map, const EnsState *st, int cold);
+void ens_friction_ab_f(hipStream_t s, const EnsMember *mem, const EnsMap &map,   const EnsState *st, int cold);
 void ens_project_f(hipStream_t s, const EnsMember *mem, const EnsMap &map, const EnsState *st, int which);
 // pint = the estimate dpr[0] (images included); then the three increments zeroed
 void ens_cold_pint(hipStream_t s, const EnsMember *mem, const EnsMap &map);

@@ -761,6 +761,98 @@ __global__ __launch_bounds__(BX * BY) void k_ab(StepConsts c, AbArgs a)
     if (a.halo) write_images<double>(c, a.dst[f], i, j, k, val, 0);
 }
 
+// biharmonic_v of several fields in one launch, and (AB) the Adams-Bashforth
+// update that follows it in a step that no forcing comes between.  A thread
+// takes BV_LEVELS levels of one column: the fluxes and second derivatives of a
+// level are formed once and serve the levels on both sides (the operands, so
+// the bits, of k_biharmonic_v).  A field with Vm = 0 passes through.
+//
+// Bound: memory (one read and one write of a field, with AB the slots too);
+// on small grids latency, which the loads of all levels in flight together
+// hide.  100x100x20: four launches of 5.0 us and the AB pass of 8.7 us become
+// one of 10.5 us.
+constexpr int BV_LEVELS = 4;
+
+struct BihvArgs {
+    AbArgs ab;              // src, dst; the rest with AB
+    double Vm[4];
+    int zero_top[4];
+};
+
+template <bool AB>
+__global__ __launch_bounds__(256) void k_bihv(StepConsts c, BihvArgs a, int nchunk)
+{
+    // AB: interior columns; else all columns, as the halo's are copied too
+    const int i = blockIdx.x * (int)blockDim.x + threadIdx.x + (AB ? 1 : -1);
+    const int j = blockIdx.y * (int)blockDim.y + threadIdx.y + (AB ? 1 : -1);
+    const int f = (int)blockIdx.z / nchunk, ch = (int)blockIdx.z % nchunk;
+    if (i > c.nx + (AB ? 0 : 2) || j > c.ny + (AB ? 0 : 2)) return;
+    const int nz = c.nz;
+    const bool lid = c.lid != 0;
+    const double Vm = a.Vm[f], dz = c.dz, rdz = c.rdz;
+    const double *in = a.ab.src[f] + idx(c, i, j, -1);
+    double *out = a.ab.dst[f] + idx(c, i, j, -1);
+    const bool zt = a.zero_top[f] != 0;
+    const int kb = 1 + ch * BV_LEVELS;
+    // v[q]: level kb - 2 + q
+    double v[BV_LEVELS + 4];
+#pragma unroll
+    for (int q = 0; q < BV_LEVELS + 4; ++q) v[q] = in[c.XY * (int64_t)min(kb - 1 + q, nz + 3)];
+    double t0[BV_LEVELS] = {}, t1[BV_LEVELS] = {}, t2[BV_LEVELS] = {};
+    if constexpr (AB) {
+#pragma unroll
+        for (int q = 0; q < BV_LEVELS; ++q) {
+            const int64_t o = idx(c, i, j, min(kb + q, nz));
+            t0[q] = a.ab.t0[f][o];
+            if (a.ab.order >= 2) t1[q] = a.ab.t1[f][o];
+            if (a.ab.order >= 3) t2[q] = a.ab.t2[f][o];
+        }
+    }
+    const bool interior = AB || (i >= 1 && i <= c.nx && j >= 1 && j <= c.ny);
+    if constexpr (!AB) {   // levels below 1 and above nz
+        if (ch == 0) {
+            out[0] = v[0];
+            out[c.XY] = v[1];
+        }
+        if (ch == nchunk - 1) {
+            out[c.XY * (int64_t)(nz + 2)] = zt ? 0.0 : in[c.XY * (int64_t)(nz + 2)];
+            out[c.XY * (int64_t)(nz + 3)] = zt ? 0.0 : in[c.XY * (int64_t)(nz + 3)];
+        }
+    }
+    auto f1 = [&](int kk, double lo, double hi) {
+        return (lid && (kk <= 0 || kk >= nz)) ? 0.0 : -div_rn(Vm * (hi - lo), dz, rdz);
+    };
+    // f1 through the upper face and del2 of the level being finished and of
+    // the one above it
+    double fu = f1(kb - 1, v[1], v[2]);
+    double dm = div_rn(fu - f1(kb - 2, v[0], v[1]), dz, rdz);
+    double fn = f1(kb, v[2], v[3]);
+    double dc = div_rn(fn - fu, dz, rdz);
+    double f20 = (lid && kb - 1 <= 0) ? 0.0 : div_rn(dc - dm, dz, rdz);
+#pragma unroll
+    for (int q = 0; q < BV_LEVELS; ++q) {
+        const int k = kb + q;
+        if (k > nz) break;
+        const double fp = f1(k + 1, v[q + 3], v[q + 4]);
+        const double dp = div_rn(fp - fn, dz, rdz);
+        const double f21 = (lid && k >= nz) ? 0.0 : div_rn(dp - dc, dz, rdz);
+        double r = v[q + 2];
+        if (interior && Vm > 0.0) r = r + c.dt * div_rn(f21 - f20, dz, rdz);
+        if (zt && k >= nz) r = 0.0;
+        if constexpr (AB) {
+            const double s = a.ab.scale[f];
+            if (a.ab.order == 1) r = r + s * t0[q];
+            else if (a.ab.order == 2) r = r + s * (a.ab.ca * t0[q] - a.ab.cb * t1[q]);
+            else r = r + s * (a.ab.ca * t0[q] + a.ab.cb * t1[q] + a.ab.cc * t2[q]);
+            if (a.ab.halo) write_images<double>(c, a.ab.dst[f], i, j, k, r, 0);
+        }
+        out[c.XY * (int64_t)(k + 1)] = r;
+        fn = fp;
+        dc = dp;
+        f20 = f21;
+    }
+}
+
 // the background forcing and the Adams-Bashforth update in one pass (a
 // forced step whose only forcing is the background flow / body force, after
 // the friction-only pass: the fields are read from the second buffers and
@@ -856,7 +948,7 @@ struct FricField {
 
 template <class T>
 struct FricArgs {
-    FricField<T> f[4];
+    FricField<T> f[4];   // a work-group's field: fric_field
     double ca, cb, cc;
     int order;
     int nchunk, kc, tiles_x, tiles_y, nblocks;
@@ -864,8 +956,18 @@ struct FricArgs {
     // u, v, w subtract scale * grad(Q) (see the step in api.hip)
     const float *d1, *d2;
     double qc1, qc2;
-    int halo;   // also write the new values' halo images (integrate.f90:106-111)
+    // HALO_IMAGES: also write the new values' halo images (integrate.f90:106-111);
+    // HALO_KEEP: out's halo takes in's values (the out-of-place friction leaves
+    // the halo that the reference's in-place passes leave); HALO_KEEP_TOP: so
+    // too, but zero from level nz on for a field with zero_top, as k_harmonic
+    // leaves it.  The copies are work-groups of their own at the end of the
+    // grid (hblocks per field): done by the tiles, the edge tiles become the
+    // slow ones and every tile pays in registers (512x128x128: 278 us; with a
+    // launch of its own 233 and 18 us; so 249 us.  FP32 202 and 16; so 188).
+    int halo, hblocks;
 };
+constexpr int HALO_PT = FRIC_HALO / FTHREADS;
+enum { HALO_NONE = 0, HALO_IMAGES = 1, HALO_KEEP = 2, HALO_KEEP_TOP = 3 };
 
 // T = double: the drop-in, bit-exact.  T = float: the mixed form -- stencils
 // in FP32, and the new state (hi + lo) + harmonic increment + biharmonic
@@ -1056,7 +1158,7 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
                 else if (a.order == 2) val = f2 + s * (a.ca * cur.s0 - a.cb * cur.s1);
                 else val = f2 + s * (a.ca * cur.s0 + a.cb * cur.s1 + a.cc * cur.s2);
                 at(F.out + lk, o2) = val;
-                if (a.halo) write_images<double>(c, F.out, i, j, k, val, 0);
+                if (a.halo == HALO_IMAGES) write_images<double>(c, F.out, i, j, k, val, 0);
             } else {
                 const double s = F.scale;
                 double ab;
@@ -1081,7 +1183,7 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
                 const float hi = (float)x;
                 at(F.out + lk, o2) = hi;
                 at(F.out_lo + lk, o2) = (float)(x - (double)hi);
-                if (a.halo) write_images<float>(c, F.out, i, j, k, hi, 0);
+                if (a.halo == HALO_IMAGES) write_images<float>(c, F.out, i, j, k, hi, 0);
             }
         }
         // no barrier here: the next level's first barrier orders this level's
@@ -1095,13 +1197,6 @@ __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T>
         level(k, pl0, pl1, pl2);
         if (++k > ke) break;
     }
-}
-
-template <class T>
-__global__ __launch_bounds__(FTHREADS, FricPlane<T>::WAVES) void k_fric_ab(StepConsts c, FricArgs<T> a)
-{
-    const int bid = xcd_remap((int)blockIdx.x, a.nblocks);
-    fric_body<T>(c, a, a.f[fric_field(a, bid)], bid);
 }
 
 // ---------------------------------------------------------------------------
@@ -1119,30 +1214,66 @@ struct HaloArgsT {
 };
 using HaloArgs = HaloArgsT<double>;
 
-// coordinates of halo point t (0 <= t < number of halo points)
-__device__ __forceinline__ void halo_ijk(const StepConsts &c, int64_t t, int &i, int &j, int &k)
+// coordinates of halo point t (0 <= t < number of halo points, which is below
+// 2^31 for every grid the FFTs take)
+__device__ __forceinline__ void halo_ijk(const StepConsts &c, int64_t t64, int &i, int &j, int &k)
 {
     const int nx = c.nx, ny = c.ny, nz = c.nz;
-    const int64_t X = c.X, Y = ny + 4;
-    const int64_t nzp = 4 * X * Y, nyr = 4 * X * (int64_t)nz;
+    const unsigned X = (unsigned)c.X, Y = (unsigned)ny + 4, t = (unsigned)t64;
+    const unsigned nzp = 4 * X * Y, nyr = 4 * X * (unsigned)nz;
     if (t < nzp) {
-        const int64_t q = t / (X * Y), r = t % (X * Y);
+        const unsigned q = t / (X * Y), r = t % (X * Y);
         k = q < 2 ? (int)q - 1 : nz + (int)q - 1;   // -1, 0, nz+1, nz+2
         j = (int)(r / X) - 1;
         i = (int)(r % X) - 1;
     } else if (t < nzp + nyr) {
-        const int64_t s = t - nzp;
-        const int64_t q = s / (X * nz), r = s % (X * nz);
+        const unsigned s = t - nzp;
+        const unsigned q = s / (X * (unsigned)nz), r = s % (X * (unsigned)nz);
         j = q < 2 ? (int)q - 1 : ny + (int)q - 1;
         k = (int)(r / X) + 1;
         i = (int)(r % X) - 1;
     } else {
-        const int64_t s = t - nzp - nyr;
-        const int64_t q = s % 4, r = s / 4;
+        const unsigned s = t - nzp - nyr;
+        const unsigned q = s % 4, r = s / 4;
         i = q < 2 ? (int)q - 1 : nx + (int)q - 1;
-        j = (int)(r % ny) + 1;
-        k = (int)(r / ny) + 1;
+        j = (int)(r % (unsigned)ny) + 1;
+        k = (int)(r / (unsigned)ny) + 1;
     }
+}
+
+// HALO_KEEP, HALO_KEEP_TOP: block hb of the halo copies of one field (hi
+// part), HALO_PT points per thread
+template <class T>
+__device__ __forceinline__ void keep_halo(const StepConsts &c, int halo, const FricField<T> &F, int hb)
+{
+    const int64_t nhalo = c.XY * (c.nz + 4) - (int64_t)c.nx * c.ny * c.nz;
+    const int64_t t0 = (int64_t)hb * (FTHREADS * HALO_PT) + threadIdx.x;
+    int64_t o[HALO_PT];
+    T v[HALO_PT];
+#pragma unroll
+    for (int s = 0; s < HALO_PT; ++s) {
+        const int64_t t = t0 + s * FTHREADS;
+        int i, j, k;
+        halo_ijk(c, min(t, nhalo - 1), i, j, k);
+        o[s] = t < nhalo ? idx(c, i, j, k) : -1;
+        v[s] = F.in[idx(c, i, j, k)];
+        if (halo == HALO_KEEP_TOP && F.zero_top && k >= c.nz) v[s] = T(0);
+    }
+#pragma unroll
+    for (int s = 0; s < HALO_PT; ++s)
+        if (o[s] >= 0) F.out[o[s]] = v[s];
+}
+
+template <class T>
+__global__ __launch_bounds__(FTHREADS, FricPlane<T>::WAVES) void k_fric_ab(StepConsts c, FricArgs<T> a)
+{
+    if ((int)blockIdx.x >= a.nblocks) {
+        const int hb = (int)blockIdx.x - a.nblocks;
+        keep_halo<T>(c, a.halo, a.f[hb / a.hblocks], hb % a.hblocks);
+        return;
+    }
+    const int bid = xcd_remap((int)blockIdx.x, a.nblocks);
+    fric_body<T>(c, a, a.f[fric_field(a, bid)], bid);
 }
 
 // halo point t (0 <= t < number of halo points) of array a
@@ -1163,26 +1294,6 @@ __global__ __launch_bounds__(256) void k_halo(StepConsts c, HaloArgsT<T> h, int6
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (t >= nhalo) return;
     halo_point<T>(c, h.f[blockIdx.y], h.neumann[blockIdx.y], t);
-}
-
-// dst's halo points take src's values (the same points): the halos of an
-// out-of-place friction result keep the pre-friction values, as the
-// reference's in-place friction leaves them
-template <class T>
-struct HaloCopyArgs {
-    const T *src[4];
-    T *dst[4];
-};
-
-template <class T>
-__global__ __launch_bounds__(256) void k_halo_copy(StepConsts c, HaloCopyArgs<T> h, int64_t nhalo)
-{
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (t >= nhalo) return;
-    int i, j, k;
-    halo_ijk(c, t, i, j, k);
-    const int64_t o = idx(c, i, j, k);
-    h.dst[blockIdx.y][o] = h.src[blockIdx.y][o];
 }
 
 // ---------------------------------------------------------------------------
@@ -1363,6 +1474,16 @@ __global__ __launch_bounds__(FTHREADS, FricPlane<double>::WAVES) void k_ens_fric
     const StepConsts c = e.c;
     const int par = st->par, itt = st->itt;
     const int lb = g - map.start[mi];
+    const int nfric = e.fric_tx * e.fric_ty * e.fric_nchunk * 4;
+    if (lb >= nfric) {   // a forced member's halo copies (see below)
+        const int per = (int)((e.H - (int64_t)c.nx * c.ny * c.nz + FRIC_HALO - 1) / FRIC_HALO);
+        const int hb = lb - nfric, f = hb / per;
+        FricField<double> F{};
+        F.in = e.f[f][par];
+        F.out = e.tmp[f];
+        keep_halo<double>(c, HALO_KEEP, F, hb % per);
+        return;
+    }
     FricArgs<double> a{};   // tiling and AB coefficients; the field record is built alone
     a.kc = e.fric_kc; a.nchunk = e.fric_nchunk; a.tiles_x = e.fric_tx; a.tiles_y = e.fric_ty;
     if (itt == 0) {
@@ -1395,36 +1516,14 @@ __global__ __launch_bounds__(FTHREADS, FricPlane<double>::WAVES) void k_ens_fric
     a.halo = 1;
     if (e.forced) {
         // set_forcing sees the post-friction state (integrate.f90:82): the
-        // friction chain alone into the third buffers; the halo copy and the
-        // forcing + AB stages follow (launch_friction_fused_only, then
-        // launch_background_ab, of a single model)
+        // friction chain alone into the third buffers; the forcing + AB stage
+        // follows (launch_friction_fused_only, then launch_background_ab, of a
+        // single model)
         a.order = 0;
         F.out = e.tmp[f];
-        a.halo = 0;
+        a.halo = HALO_KEEP;
     }
     fric_body<double>(c, a, F, lb);
-}
-
-// forced members: the third buffers' halos take the pre-friction values (the
-// halo the reference's in-place friction leaves), k_halo_copy per member
-__global__ __launch_bounds__(256) void k_ens_halo_copy(const EnsMember *__restrict__ mem, EnsMap map,
-                                                        const EnsState *__restrict__ st, int mixed)
-{
-    const int g = xcd_remap((int)blockIdx.x, map.start[map.n]);
-    const int mi = ens_find(map, g);
-    const EnsMember &e = mem[mi];
-    const StepConsts c = e.c;
-    const int64_t nhalo = e.H - (int64_t)c.nx * c.ny * c.nz;
-    const int64_t per = (nhalo + 255) / 256;
-    const int64_t lb = g - map.start[mi];
-    const int f = (int)(lb / per);
-    const int64_t t = (lb % per) * 256 + threadIdx.x;
-    if (f > 3 || t >= nhalo) return;
-    int i, j, k;
-    halo_ijk(c, t, i, j, k);
-    const int64_t o = idx(c, i, j, k);
-    if (mixed) e.tmph[f][o] = e.fh[f][st->par][o];   // the hi parts (halo_copy<float>)
-    else e.tmp[f][o] = e.f[f][st->par][o];
 }
 
 // forced members: background flow / body force and the Adams-Bashforth
@@ -1659,6 +1758,17 @@ __global__ __launch_bounds__(FTHREADS, FricPlane<float>::WAVES) void k_ens_fric_
     const StepConsts c = e.c;
     const int par = st->par, itt = cold ? 0 : st->itt, cur = st->dp_cur;
     const int lb = g - map.start[mi];
+    const int nfric = e.fric_tx * e.fric_ty * e.fric_nchunk * 4;
+    if (lb >= nfric) {   // a forced member's halo copies (see below)
+        if (cold) return;
+        const int per = (int)((e.H - (int64_t)c.nx * c.ny * c.nz + FRIC_HALO - 1) / FRIC_HALO);
+        const int hb = lb - nfric, f = hb / per;
+        FricField<float> F{};
+        F.in = e.fh[f][par];
+        F.out = e.tmph[f];
+        keep_halo<float>(c, HALO_KEEP, F, hb % per);
+        return;
+    }
     FricArgs<float> a{};
     a.kc = e.fric_kc; a.nchunk = e.fric_nchunk; a.tiles_x = e.fric_tx; a.tiles_y = e.fric_ty;
     double qc1 = 0.0, qc2 = 0.0;
@@ -1705,13 +1815,13 @@ __global__ __launch_bounds__(FTHREADS, FricPlane<float>::WAVES) void k_ens_fric_
     if (e.forced && !cold) {
         // the forcing sees the post-friction state: friction alone into the
         // third (hi, lo) buffers (launch_friction_forcing_ab_mixed of a
-        // single model); the halo copy and forcing + AB stages follow
+        // single model); the forcing + AB stage follows
         a.order = 0;
         a.qc1 = a.qc2 = 0.0;
         a.d1 = a.d2 = nullptr;
         F.out = e.tmph[f];
         F.out_lo = e.tmpl[f];
-        a.halo = 0;
+        a.halo = HALO_KEEP;
     }
     fric_body<float>(c, a, F, lb);
 }
@@ -1808,16 +1918,28 @@ inline dim3 march_grid(const Grid &g, int &kc)
     return dim3((unsigned)((g.nx + BX - 1) / BX), (unsigned)((g.ny + BY - 1) / BY), (unsigned)nch);
 }
 
-// Levels per work-group of the tendency kernel: at least 512 work-groups (two
-// per CU) where the grid has the levels for it, of at most 16 levels.  On
-// small grids a work-group's levels are one after the other on an idle chip:
-// 64x64x32, 9.6 us with 1 level, 14.5 with 4, 21.9 with 8; 120x120x10, 10.7
-// with 1, 25 with 10; 160x120x37, 20 with 4, 31 with 13.  On large ones
-// 512x512x64 takes 250 us with 16 levels, 262 with 64.
+// Levels per work-group of the tendency kernel, up to 16: the fewest rounds of
+// 512 work-groups (two per CU) times the levels of each and the four or so
+// that a work-group's start costs.  On small grids a work-group's levels are
+// one after the other on an idle chip: 64x64x32, 8.6 us with 1 level, 11.5
+// with 4, 16.0 with 8; 100x100x20, 11.1 with 2 (260 work-groups), 12.3 with 1
+// (520), 18.5 with 10.  A round that is nearly empty costs as much as a full
+// one: 192x192x40, 23.8 us with 6 levels (504 work-groups), 28.3 with 5 (576).
+// On large grids 512x512x64 takes 253 us with 16 levels, 272 with 32, and
+// 256x256x64 56 with 16, 62 with 8.
 int tendency_levels(int tiles, int nz)
 {
-    const int nchunk = std::min(nz, std::max((nz + 15) / 16, (512 + tiles - 1) / tiles));
-    return (nz + nchunk - 1) / nchunk;
+    int best = 1;
+    int64_t least = INT64_MAX;
+    for (int kc = 1; kc <= std::min(nz, 16); ++kc) {
+        const int64_t n = (int64_t)tiles * ((nz + kc - 1) / kc);
+        const int64_t cost = (n + 511) / 512 * (kc + 4);
+        if (cost < least) {
+            least = cost;
+            best = kc;
+        }
+    }
+    return best;
 }
 
 // Levels per work-group of the friction kernel: at least 1024 work-groups
@@ -1927,31 +2049,6 @@ void launch_mixing(Model &m, int op, int f, double hmix, double vmix, int zero_t
     }
     PS3D_HIP_CHECK(hipGetLastError());
     m.cur[f] ^= 1;
-}
-
-// integrate.f90:59-78
-void launch_friction_block(Model &m)
-{
-    const ps3d_params &p = m.prm;
-    const int lid = p.enable_vertical_boundaries;
-    if (p.Ah > 0. || p.Av > 0.) {
-        launch_mixing(m, PS3D_HARMONIC, PS3D_U, p.Ah, p.Av, 0);
-        launch_mixing(m, PS3D_HARMONIC, PS3D_V, p.Ah, p.Av, 0);
-        launch_mixing(m, PS3D_HARMONIC, PS3D_W, p.Ah, p.Av, lid);
-    }
-    if (p.Kh > 0. || p.Kv > 0.) launch_mixing(m, PS3D_HARMONIC, PS3D_B, p.Kh, p.Kv, 0);
-    if (p.Ahbi > 0.) {
-        launch_mixing(m, PS3D_BIHARMONIC_H, PS3D_U, p.Ahbi, 0.0, 0);
-        launch_mixing(m, PS3D_BIHARMONIC_H, PS3D_V, p.Ahbi, 0.0, 0);
-        launch_mixing(m, PS3D_BIHARMONIC_H, PS3D_W, p.Ahbi, 0.0, 0);
-    }
-    if (p.Avbi > 0.) {
-        launch_mixing(m, PS3D_BIHARMONIC_V, PS3D_U, 0.0, p.Avbi, 0);
-        launch_mixing(m, PS3D_BIHARMONIC_V, PS3D_V, 0.0, p.Avbi, 0);
-        launch_mixing(m, PS3D_BIHARMONIC_V, PS3D_W, 0.0, p.Avbi, lid);
-    }
-    if (p.Khbi > 0.) launch_mixing(m, PS3D_BIHARMONIC_H, PS3D_B, p.Khbi, 0.0, 0);
-    if (p.Kvbi > 0.) launch_mixing(m, PS3D_BIHARMONIC_V, PS3D_B, 0.0, p.Kvbi, 0);
 }
 
 static BgArgs<double> bg_args(Model &m, int tau)
@@ -2095,12 +2192,14 @@ bool fused_friction_ok(const Model &m)
 // writes the new values' halo images (the exchange of integrate.f90:106-111).
 // The new fields are written to the second buffers, which then become the
 // canonical ones.
-// itt < 0: friction only (no AB).  halo: write the new values' halo images
-// (-1: where the model does, fuse_halo)
+// itt < 0: friction only (no AB).  halo: the HALO_ mode (-1: images where the
+// model's kernels write them, fuse_halo).  fields: the fields that take part
+// (bit f)
 template <class T>
 static void friction_ab_impl(Model &m, const T *const *in, const T *const *in_lo, T *const *out, T *const *out_lo,
                              T *const *tend, int itt, int tau, int taum1, int taum2, double qc1 = 0.0,
-                             const float *d1 = nullptr, double qc2 = 0.0, const float *d2 = nullptr, int halo = -1)
+                             const float *d1 = nullptr, double qc2 = 0.0, const float *d2 = nullptr, int halo = -1,
+                             unsigned fields = 15)
 {
     const ps3d_params &p = m.prm;
     const Grid &g = m.g;
@@ -2109,8 +2208,10 @@ static void friction_ab_impl(Model &m, const T *const *in, const T *const *in_lo
     a.d2 = d2;
     a.qc1 = qc1;
     a.qc2 = qc2;
+    int nf = 0;
     for (int f = 0; f < 4; ++f) {
-        FricField<T> &F = a.f[f];
+        if (!(fields >> f & 1)) continue;
+        FricField<T> &F = a.f[nf++];
         F.in = in[f];
         F.in_lo = in_lo ? in_lo[f] : nullptr;
         F.out = out[f];
@@ -2155,26 +2256,12 @@ static void friction_ab_impl(Model &m, const T *const *in, const T *const *in_lo
     const int tiles = a.tiles_x * a.tiles_y;
     a.kc = m.fric_kc > 0 ? m.fric_kc : friction_levels(tiles, g.nz, std::is_same<T, float>::value);
     a.nchunk = (g.nz + a.kc - 1) / a.kc;
-    a.nblocks = tiles * a.nchunk * 4;
-    a.halo = halo < 0 ? (m.fuse_halo ? 1 : 0) : halo;
+    a.nblocks = tiles * a.nchunk * nf;
+    a.halo = halo < 0 ? (m.fuse_halo ? HALO_IMAGES : HALO_NONE) : halo;
+    a.hblocks = a.halo >= HALO_KEEP ? (int)((g.H - g.N + FRIC_HALO - 1) / FRIC_HALO) : 0;
     ProfScope ps(m, "friction_ab");
-    hipLaunchKernelGGL(k_fric_ab<T>, dim3((unsigned)a.nblocks), dim3(FTHREADS), 0, m.stream, m.c, a);
-    PS3D_HIP_CHECK(hipGetLastError());
-}
-
-// the halo points of four arrays copied into four others
-template <class T>
-static void halo_copy(Model &m, const T *const *src, T *const *dst)
-{
-    HaloCopyArgs<T> h{};
-    for (int f = 0; f < 4; ++f) {
-        h.src[f] = src[f];
-        h.dst[f] = dst[f];
-    }
-    const int64_t nhalo = m.g.H - m.g.N;
-    ProfScope ps(m, "halo");
-    hipLaunchKernelGGL(k_halo_copy<T>, dim3((unsigned)((nhalo + 255) / 256), 4), dim3(256), 0, m.stream, m.c, h,
-                       nhalo);
+    const unsigned nb = (unsigned)(a.nblocks + a.hblocks * nf);
+    hipLaunchKernelGGL(k_fric_ab<T>, dim3(nb), dim3(FTHREADS), 0, m.stream, m.c, a);
     PS3D_HIP_CHECK(hipGetLastError());
 }
 
@@ -2186,6 +2273,99 @@ static void halo_launch(Model &m, const HaloArgsT<T> &h, int n)
     hipLaunchKernelGGL(k_halo<T>, dim3((unsigned)((nhalo + 255) / 256), (unsigned)n), dim3(256), 0, m.stream, m.c,
                        h, nhalo);
     PS3D_HIP_CHECK(hipGetLastError());
+}
+
+// the harmonic and biharmonic_h operators of integrate.f90:59-78, of all
+// fields in one launch into the buffers that are not current, halos included.
+// For a field their order is that of the reference; between fields nothing
+// passes.
+static void friction_tiled(Model &m)
+{
+    const ps3d_params &p = m.prm;
+    double *in[4], *out[4];
+    double *tend[4] = {m.du, m.dv, m.dw, m.db};
+    unsigned fields = 0;
+    for (int f = 0; f < 4; ++f) {
+        in[f] = m.cur_buf(f);
+        out[f] = m.cur[f] ? m.field_buf(f) : m.alt[f];
+        const bool on = f < 3 ? (p.Ah > 0. || p.Av > 0. || p.Ahbi > 0.) : (p.Kh > 0. || p.Kv > 0. || p.Khbi > 0.);
+        if (on) fields |= 1u << f;
+    }
+    if (!fields) return;
+    friction_ab_impl<double>(m, in, nullptr, out, nullptr, tend, -1, 1, 2, 3, 0.0, nullptr, 0.0, nullptr,
+                             HALO_KEEP_TOP, fields);
+    for (int f = 0; f < 4; ++f) m.cur[f] ^= fields >> f & 1;
+}
+
+static BihvArgs bihv_args(const Model &m)
+{
+    BihvArgs a{};
+    for (int f = 0; f < 4; ++f) a.Vm[f] = f < 3 ? m.prm.Avbi : m.prm.Kvbi;
+    a.zero_top[2] = a.Vm[2] > 0. && m.prm.enable_vertical_boundaries;
+    return a;
+}
+
+// biharmonic_v of the fields that have it, into the buffers that are not current
+static void launch_bihv(Model &m)
+{
+    const BihvArgs v = bihv_args(m);
+    BihvArgs a{};
+    int n = 0;
+    for (int f = 0; f < 4; ++f) {
+        if (!(v.Vm[f] > 0.)) continue;
+        a.Vm[n] = v.Vm[f];
+        a.zero_top[n] = v.zero_top[f];
+        a.ab.src[n] = m.cur_buf(f);
+        a.ab.dst[n] = m.cur[f] ? m.field_buf(f) : m.alt[f];
+        m.cur[f] ^= 1;
+        ++n;
+    }
+    if (!n) return;
+    const Grid &g = m.g;
+    const int nchunk = (g.nz + BV_LEVELS - 1) / BV_LEVELS;
+    ProfScope ps(m, "biharmonic_v");
+    hipLaunchKernelGGL(k_bihv<false>,
+                       dim3((unsigned)((g.X + BX - 1) / BX), (unsigned)((g.Y + BY - 1) / BY), (unsigned)(nchunk * n)),
+                       dim3(BX, BY), 0, m.stream, m.c, a, nchunk);
+    PS3D_HIP_CHECK(hipGetLastError());
+}
+
+// integrate.f90:59-78.  One launch for the harmonic and biharmonic_h
+// operators and one for biharmonic_v: harmonic and biharmonic_h of four fields
+// one by one are eight launches and 64 us at 160x120x37, this one 38 us; at
+// 100x100x20 37 and 16 us.
+void launch_friction_block(Model &m)
+{
+    friction_tiled(m);
+    launch_bihv(m);
+}
+
+// integrate.f90:59-111 with vertical biharmonic friction and no forcing: the
+// tiled friction, then biharmonic_v and the AB update in one pass from the
+// second buffers into the canonical ones (which other threads still read
+// where no tiled operator moved a field: then the passes stay apart)
+void launch_friction_block_ab(Model &m, int itt, int tau, int taum1, int taum2)
+{
+    friction_tiled(m);
+    BihvArgs a = bihv_args(m);
+    bool fuse = true;
+    for (int f = 0; f < 4; ++f)
+        if (a.Vm[f] > 0. && !m.cur[f]) fuse = false;
+    if (!fuse) {
+        launch_bihv(m);
+        launch_ab_exchange(m, itt, tau, taum1, taum2);
+        return;
+    }
+    a.ab = ab_args(m, itt, tau, taum1, taum2);
+    const int nchunk = (m.g.nz + BV_LEVELS - 1) / BV_LEVELS;
+    {
+        ProfScope ps(m, "ab_update");
+        PointShape sh = point_shape(m.g);
+        sh.grid.z = (unsigned)(nchunk * 4);
+        hipLaunchKernelGGL(k_bihv<true>, sh.grid, sh.block, 0, m.stream, m.c, a, nchunk);
+        PS3D_HIP_CHECK(hipGetLastError());
+    }
+    ab_finish(m);
 }
 
 // integrate.f90:59-111 for configs without vertical biharmonic friction:
@@ -2219,10 +2399,10 @@ void launch_friction_ab_mixed(Model &m, int itt, int tau, int taum1, int taum2, 
 void launch_friction_forcing_ab_mixed(Model &m, int itt, int tau, int taum1, int taum2, double qc1, const float *d1,
                                       double qc2, const float *d2)
 {
-    // interior only (halo 0); the hi halos take the pre-friction values, which
-    // the forcing reads (the lo parts and the AB pass use interior points only)
-    friction_ab_impl<float>(m, m.fh, m.fl, m.ah, m.al, m.tf, -1, tau, taum1, taum2, 0.0, nullptr, 0.0, nullptr, 0);
-    halo_copy<float>(m, m.fh, m.ah);
+    // the hi halos take the pre-friction values, which the forcing reads (the
+    // lo parts and the AB pass use interior points only)
+    friction_ab_impl<float>(m, m.fh, m.fl, m.ah, m.al, m.tf, -1, tau, taum1, taum2, 0.0, nullptr, 0.0, nullptr,
+                            HALO_KEEP);
     launch_background(m, tau, m.ah);
     AbMixedArgs a{};
     const ps3d_params &p = m.prm;
@@ -2269,7 +2449,7 @@ void launch_friction_forcing_ab_mixed(Model &m, int itt, int tau, int taum1, int
 // autotuner's timing launch
 // integrate.f90:59-78 for a forced FP64 step without vertical biharmonic
 // friction: the fused kernel's friction chain alone (no AB) into the second
-// buffers, whose halos then take the pre-friction values; the forcing and
+// buffers, whose halos take the pre-friction values; the forcing and
 // the Adams-Bashforth pass (launch_ab_exchange) read the second buffers
 void launch_friction_fused_only(Model &m)
 {
@@ -2277,8 +2457,8 @@ void launch_friction_fused_only(Model &m)
     double *in[4] = {m.field_buf(0), m.field_buf(1), m.field_buf(2), m.field_buf(3)};
     double *out[4] = {m.alt[0], m.alt[1], m.alt[2], m.alt[3]};
     double *tend[4] = {m.du, m.dv, m.dw, m.db};
-    friction_ab_impl<double>(m, in, nullptr, out, nullptr, tend, -1, 1, 2, 3, 0.0, nullptr, 0.0, nullptr, 0);
-    halo_copy<double>(m, in, out);
+    friction_ab_impl<double>(m, in, nullptr, out, nullptr, tend, -1, 1, 2, 3, 0.0, nullptr, 0.0, nullptr,
+                             HALO_KEEP);
     for (int f = 0; f < 4; ++f) m.cur[f] = 1;
 }
 
@@ -2391,14 +2571,6 @@ void ens_friction_ab(hipStream_t s, const EnsMember *mem, const EnsMap &map, con
 {
     if (!map.start[map.n]) return;
     hipLaunchKernelGGL(k_ens_fric, dim3((unsigned)map.start[map.n]), dim3(FTHREADS), 0, s, mem, map, st);
-    PS3D_HIP_CHECK(hipGetLastError());
-}
-
-void ens_halo_copy(hipStream_t s, const EnsMember *mem, const EnsMap &map, const EnsState *st, bool mixed)
-{
-    if (!map.start[map.n]) return;
-    hipLaunchKernelGGL(k_ens_halo_copy, dim3((unsigned)map.start[map.n]), dim3(256), 0, s, mem, map, st,
-                       mixed ? 1 : 0);
     PS3D_HIP_CHECK(hipGetLastError());
 }
 

@@ -186,7 +186,7 @@ void tune_model(Model &m, int next_tau, const char *cache_path, int reps)
         if (m.mixed) launch_tendency_mixed(m, next_tau, m.pint);
         else launch_tendency(m, next_tau);
     });
-    if (m.mixed || (fused_friction_ok(m) && m.fuse_friction))
+    if (m.mixed || (fused_friction_ok(m)))
         pick("friction_ab", levels, m.fric_kc, reps, nullptr,
              [&] { launch_friction_ab_raw(m, 3, next_tau, t1, t2); });
     if (m.mixed) {

@@ -60,3 +60,65 @@ def test_mixed_step(size):
         assert err[k] <= 1e-5, (k, err[k])
     gpu.close()
     orc.close()
+
+
+OPS = {
+    "all": {},
+    "vertical_only": dict(Ah=0.0, Av=0.0, Kh=0.0, Kv=0.0, Ahbi=0.0, Khbi=0.0),
+    "harmonic_and_vertical_of_uvw": dict(Ahbi=0.0, Khbi=0.0, Kh=0.0, Kv=0.0, Kvbi=0.0),
+    "biharmonic_of_b": dict(Ah=0.0, Av=0.0, Ahbi=0.0, Avbi=0.0, Kh=0.0, Kv=0.0),
+}
+
+
+@pytest.mark.parametrize("lid", [True, False])
+@pytest.mark.parametrize("ops", list(OPS))
+@pytest.mark.parametrize("size", [(2, 2, 2), (4, 4, 4), (30, 10, 5), (64, 8, 9), (128, 18, 12)])
+def test_friction_block_bitwise(size, ops, lid):
+    """The friction operators in their launches (two, where the halo can be
+    carried along) against the oracle's single ones, twice in a row, halo
+    included -- a halo that is not the interior's image."""
+    from ps3d_amd import configs
+    nx, ny, nz = size
+    if not lid:
+        nz += nz % 2
+    print(f"friction {nx}x{ny}x{nz} {ops} lid={lid}", flush=True)
+    prm, gpu, orc = _pair(configs.random_state(nx, ny, nz, lid=lid, **OPS[ops]))
+    rng = np.random.default_rng(3)
+    for n in ("u", "v", "w", "b"):
+        a = gpu.f[n] + 1e-3 * rng.standard_normal(gpu.f[n].shape)
+        gpu.f[n][...] = a
+        orc.f[n][...] = a
+    gpu.push(["u", "v", "w", "b"])
+    for _ in range(2):
+        gpu.friction()
+        for n in ("u", "v", "w", "b"):
+            H, V, Hb, Vb = (prm.Ah, prm.Av, prm.Ahbi, prm.Avbi) if n != "b" else (prm.Kh, prm.Kv, prm.Khbi, prm.Kvbi)
+            if H > 0 or V > 0:
+                orc.harmonic(n, H, V)
+                if n == "w" and lid:
+                    orc.f["w"][:, :, nz + 1:] = 0.0   # integrate.f90:63
+            if Hb > 0:
+                orc.biharmonic_h(n, Hb)
+            if Vb > 0:
+                orc.biharmonic_v(n, Vb)
+                if n == "w" and lid:
+                    orc.f["w"][:, :, nz + 1:] = 0.0   # integrate.f90:73
+        gpu.pull(["u", "v", "w", "b"])
+        for n in ("u", "v", "w", "b"):
+            assert np.array_equal(gpu.f[n], orc.f[n]), n
+    gpu.close()
+    orc.close()
+
+
+@pytest.mark.parametrize("ops", list(OPS))
+def test_steps_with_vertical_friction_bitwise(ops):
+    from ps3d_amd import configs
+    print(f"steps {ops}", flush=True)
+    prm, gpu, orc = _pair(configs.random_state(72, 10, 13, lid=True, **OPS[ops]))
+    gpu.run(4)
+    orc.run(4)
+    gpu.pull()
+    for n in ("u", "v", "w", "b", "p"):
+        assert np.array_equal(gpu.f[n], orc.f[n]), n
+    gpu.close()
+    orc.close()
