@@ -451,14 +451,20 @@ constexpr Fac factorize(int N, int PL)
     return F;
 }
 
-// one Stockham pass; element e of column col at buf[e*ES + col*CS]
-template <int R, int N, int NS, int NCOL, int T, int ES, int CS, bool COLFAST, int SIGN, class C>
-__device__ __forceinline__ void pass(C *buf, const C *__restrict__ tw)
+// One Stockham pass; element e of column col at buf[e*ES + col*CS].  The
+// first pass takes its inputs from src(e, col), the last gives its outputs to
+// sink(e, col, value): a transform's data go from global memory to registers
+// and from registers to global memory, and see LDS only between passes.
+// SRC_LDS: src reads buf; SINK_LDS: sink writes it.
+template <int R, int N, int NS, int NCOL, int T, int ES, int CS, bool COLFAST, int SIGN, bool SRC_LDS, bool SINK_LDS,
+          class C, class SRC, class SINK>
+__device__ __forceinline__ void pass(C *buf, const C *__restrict__ tw, SRC src, SINK sink)
 {
     constexpr int NB = N / R;
     constexpr int TOTAL = NB * NCOL;
     constexpr int PER = (TOTAL + T - 1) / T;
     constexpr int TWS = N / (NS * R);
+    constexpr bool FIRST = NS == 1, LAST = NS * R == N;
     C v[PER][R];
 #pragma unroll
     for (int s = 0; s < PER; ++s) {
@@ -467,7 +473,17 @@ __device__ __forceinline__ void pass(C *buf, const C *__restrict__ tw)
             const int col = COLFAST ? t % NCOL : t / NB;
             const int jb = COLFAST ? t / NCOL : t % NB;
 #pragma unroll
-            for (int r = 0; r < R; ++r) v[s][r] = buf[(jb + r * NB) * ES + col * CS];
+            for (int r = 0; r < R; ++r) {
+                if constexpr (FIRST) v[s][r] = src(jb + r * NB, col);
+                else v[s][r] = buf[(jb + r * NB) * ES + col * CS];
+            }
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < PER; ++s) {
+        const int t = (int)threadIdx.x + s * T;
+        if (TOTAL % T == 0 || t < TOTAL) {
+            const int jb = COLFAST ? t / NCOL : t % NB;
             if constexpr (NS > 1) {
                 const int jm = jb % NS;
 #pragma unroll
@@ -480,7 +496,7 @@ __device__ __forceinline__ void pass(C *buf, const C *__restrict__ tw)
             dftc<R, SIGN>(v[s]);
         }
     }
-    __syncthreads();
+    if constexpr ((!FIRST || SRC_LDS) && (!LAST || SINK_LDS)) __syncthreads();
 #pragma unroll
     for (int s = 0; s < PER; ++s) {
         const int t = (int)threadIdx.x + s * T;
@@ -490,27 +506,40 @@ __device__ __forceinline__ void pass(C *buf, const C *__restrict__ tw)
             const int jm = jb % NS;
             const int base = (jb / NS) * NS * R + jm;
 #pragma unroll
-            for (int r = 0; r < R; ++r) buf[(base + r * NS) * ES + col * CS] = v[s][r];
+            for (int r = 0; r < R; ++r) {
+                if constexpr (LAST) sink(base + r * NS, col, v[s][r]);
+                else buf[(base + r * NS) * ES + col * CS] = v[s][r];
+            }
         }
     }
-    __syncthreads();
+    if constexpr (!LAST || SINK_LDS) __syncthreads();
 }
 
-template <int N, int P, int NS, int NCOL, int T, int ES, int CS, bool COLFAST, int SIGN, int PL, class C>
-__device__ __forceinline__ void passes(C *buf, const C *__restrict__ tw)
+template <int N, int P, int NS, int NCOL, int T, int ES, int CS, bool COLFAST, int SIGN, int PL, bool SRC_LDS,
+          bool SINK_LDS, class C, class SRC, class SINK>
+__device__ __forceinline__ void passes(C *buf, const C *__restrict__ tw, SRC src, SINK sink)
 {
     constexpr Fac F = factorize(N, PL);
     if constexpr (P < F.n) {
         constexpr int R = F.f[P];
-        pass<R, N, NS, NCOL, T, ES, CS, COLFAST, SIGN>(buf, tw);
-        passes<N, P + 1, NS * R, NCOL, T, ES, CS, COLFAST, SIGN, PL>(buf, tw);
+        pass<R, N, NS, NCOL, T, ES, CS, COLFAST, SIGN, SRC_LDS, SINK_LDS>(buf, tw, src, sink);
+        passes<N, P + 1, NS * R, NCOL, T, ES, CS, COLFAST, SIGN, PL, SRC_LDS, SINK_LDS>(buf, tw, src, sink);
     }
 }
 
-template <int N, int NCOL, int T, int ES, int CS, bool COLFAST, int SIGN, int PL = 0, class C>
-__device__ __forceinline__ void fft(C *buf, const C *__restrict__ tw)
+// where src reads buf, a barrier lies before the call
+template <int N, int NCOL, int T, int ES, int CS, bool COLFAST, int SIGN, int PL, bool SRC_LDS, bool SINK_LDS, class C,
+          class SRC, class SINK>
+__device__ __forceinline__ void fft(C *buf, const C *__restrict__ tw, SRC src, SINK sink)
 {
-    passes<N, 0, 1, NCOL, T, ES, CS, COLFAST, SIGN, PL>(buf, tw);
+    passes<N, 0, 1, NCOL, T, ES, CS, COLFAST, SIGN, PL, SRC_LDS, SINK_LDS>(buf, tw, src, sink);
+}
+
+// two reals that lie side by side, at a multiple of their size together
+template <class RT>
+__device__ __forceinline__ typename cplx_of<RT>::type pair_at(const RT *p)
+{
+    return *reinterpret_cast<const typename cplx_of<RT>::type *>(p);
 }
 
 // x-pass, forward r2c of ROWS rows (see k_r2c_x); the post-processing works
@@ -527,35 +556,34 @@ __device__ __forceinline__ void r2c_body(typename cplx_of<RT>::type *lds, int bl
     constexpr int CS = N2 + 1;
     const int64_t row0 = (int64_t)blk * ROWS;
     const RT h = RT(0.5);
+    // z[m] = x[2m] + i x[2m+1].  A field's points 2m + 1 and 2m + 2 are one
+    // aligned pair (point i is element i + 1 of its row, rows are even)
+    auto src_z = [&](int m, int rr) {
+        const int64_t row = row0 + rr;
+        if (row >= nrows) return mk<C>(RT(0), RT(0));
+        if constexpr (FUSE_DIV) {
+            const int j = (int)((unsigned)row % (unsigned)c.ny) + 1, k = (int)((unsigned)row / (unsigned)c.ny) + 1;
+            const int64_t X = c.X, XY = c.XY;
+            const int64_t o = fidx(c, 2 * m + 1, j, k);
+            const C u1 = pair_at(u + o), v1 = pair_at(v + o), v0 = pair_at(v + o - X), w1 = pair_at(w + o),
+                    w0 = pair_at(w + o - XY);
+            RT a0 = sdiv<RT>(u1.x - u[o - 1], c.dx, c.rdx) + sdiv<RT>(v1.x - v0.x, c.dy, c.rdy) +
+                    sdiv<RT>(w1.x - w0.x, c.dz, c.rdz);
+            RT a1 = sdiv<RT>(u1.y - u1.x, c.dx, c.rdx) + sdiv<RT>(v1.y - v0.y, c.dy, c.rdy) +
+                    sdiv<RT>(w1.y - w0.y, c.dz, c.rdz);
+            return mk<C>(sdiv<RT>(a0, c.dt, c.rdt), sdiv<RT>(a1, c.dt, c.rdt));
+        } else {
+            return mk<C>(src[row * (2 * (int64_t)N2) + 2 * m], src[row * (2 * (int64_t)N2) + 2 * m + 1]);
+        }
+    };
 #pragma unroll
     for (int s = 0; s < (ROWS * N2 + T - 1) / T; ++s) {
         const int t = (int)threadIdx.x + s * T;
-        if ((ROWS * N2) % T == 0 || t < ROWS * N2) {
-            const int rr = t / N2, m = t % N2;
-            const int64_t row = row0 + rr;
-            RT a0 = RT(0), a1 = RT(0);
-            if (row < nrows) {
-                if (FUSE_DIV) {
-                    const int j = (int)(row % c.ny) + 1, k = (int)(row / c.ny) + 1;
-                    const int64_t X = c.X, XY = c.XY;
-                    int64_t o = fidx(c, 2 * m + 1, j, k);
-                    a0 = sdiv<RT>(u[o] - u[o - 1], c.dx, c.rdx) + sdiv<RT>(v[o] - v[o - X], c.dy, c.rdy) +
-                         sdiv<RT>(w[o] - w[o - XY], c.dz, c.rdz);
-                    o += 1;
-                    a1 = sdiv<RT>(u[o] - u[o - 1], c.dx, c.rdx) + sdiv<RT>(v[o] - v[o - X], c.dy, c.rdy) +
-                         sdiv<RT>(w[o] - w[o - XY], c.dz, c.rdz);
-                    a0 = sdiv<RT>(a0, c.dt, c.rdt);
-                    a1 = sdiv<RT>(a1, c.dt, c.rdt);
-                } else {
-                    a0 = src[row * (2 * (int64_t)N2) + 2 * m];
-                    a1 = src[row * (2 * (int64_t)N2) + 2 * m + 1];
-                }
-            }
-            lds[rr * CS + m] = mk<C>(a0, a1);
-        }
+        if ((ROWS * N2) % T == 0 || t < ROWS * N2) lds[t / N2 * CS + t % N2] = src_z(t % N2, t / N2);
     }
     __syncthreads();
-    fft<N2, ROWS, T, 1, CS, false, -1, PL>(lds, tw);
+    fft<N2, ROWS, T, 1, CS, false, -1, PL, true, true>(
+        lds, tw, [&](int m, int rr) { return lds[rr * CS + m]; }, [&](int m, int rr, C z) { lds[rr * CS + m] = z; });
     constexpr int HALF = N2 / 2 + 1;   // k = 0..N2/2 handles (k, N2-k)
 #pragma unroll
     for (int s = 0; s < (ROWS * HALF + T - 1) / T; ++s) {
@@ -611,6 +639,8 @@ __device__ __forceinline__ void c2r_body(typename cplx_of<RT>::type *lds, int bl
     using C = typename cplx_of<RT>::type;
     constexpr int CS = N2 + 1;
     constexpr int HALF = N2 / 2 + 1;
+    // Z'[k] = (X[k] + conj(X[N2-k])) + i conj(W^k) (X[k] - conj(X[N2-k])):
+    // the pair (k, N2 - k) at once, so that each value is read once
 #pragma unroll
     for (int s = 0; s < (ROWS * HALF + T - 1) / T; ++s) {
         const int t = (int)threadIdx.x + s * T;
@@ -641,28 +671,19 @@ __device__ __forceinline__ void c2r_body(typename cplx_of<RT>::type *lds, int bl
         }
     }
     __syncthreads();
-    fft<N2, ROWS, T, 1, CS, false, +1, PL>(lds, tw);
-#pragma unroll
-    for (int s = 0; s < (ROWS * N2 + T - 1) / T; ++s) {
-        const int t = (int)threadIdx.x + s * T;
-        if ((ROWS * N2) % T == 0 || t < ROWS * N2) {
-            const int rr = t / N2, m = t % N2;
-            const int64_t row = (int64_t)blk * ROWS + rr;
-            if (row < nrows) {
-                const C z = lds[rr * CS + m];
-                const RT a0 = sdiv<RT>(z.x, inv_scale, rinv_scale), a1 = sdiv<RT>(z.y, inv_scale, rinv_scale);
-                if (dst_is_field) {
-                    const int j = (int)(row % c.ny) + 1, k = (int)(row / c.ny) + 1;
-                    const int64_t o = fidx(c, 2 * m + 1, j, k);
-                    dst[o] = a0;
-                    dst[o + 1] = a1;
-                } else {
-                    dst[row * (2 * (int64_t)N2) + 2 * m] = a0;
-                    dst[row * (2 * (int64_t)N2) + 2 * m + 1] = a1;
-                }
-            }
+    auto put = [&](int m, int rr, C z) {
+        const int64_t row = (int64_t)blk * ROWS + rr;
+        if (row >= nrows) return;
+        const C x = mk<C>(sdiv<RT>(z.x, inv_scale, rinv_scale), sdiv<RT>(z.y, inv_scale, rinv_scale));
+        if (dst_is_field) {   // an aligned pair, see r2c_body
+            const int j = (int)((unsigned)row % (unsigned)c.ny) + 1, k = (int)((unsigned)row / (unsigned)c.ny) + 1;
+            *reinterpret_cast<C *>(dst + fidx(c, 2 * m + 1, j, k)) = x;
+        } else {
+            dst[row * (2 * (int64_t)N2) + 2 * m] = x.x;
+            dst[row * (2 * (int64_t)N2) + 2 * m + 1] = x.y;
         }
-    }
+    };
+    fft<N2, ROWS, T, 1, CS, false, +1, PL, true, false>(lds, tw, [&](int m, int rr) { return lds[rr * CS + m]; }, put);
 }
 
 template <int N2, int ROWS, int T, class RT, int PL = 0>
@@ -687,30 +708,15 @@ __device__ __forceinline__ void cols_body(C *lds, int bx, int by, const C *__res
     const int kx0 = bx * TX;
     const int ncol = min(TX, nkx - kx0);
     C *base = data + kx0 + (int64_t)by * lstride;
-#pragma unroll
-    for (int s = 0; s < (N * TX + T - 1) / T; ++s) {
-        const int t = (int)threadIdx.x + s * T;
-        if ((N * TX) % T == 0 || t < N * TX) {
-            const int col = t % TX, e = t / TX;
-            lds[e * TX + col] = (col < ncol) ? base[col + e * estride] : mk<C>(RT(0), RT(0));
-        }
-    }
-    __syncthreads();
-    fft<N, TX, T, TX, 1, true, SIGN, PL>(lds, tw);
-#pragma unroll
-    for (int s = 0; s < (N * TX + T - 1) / T; ++s) {
-        const int t = (int)threadIdx.x + s * T;
-        if ((N * TX) % T == 0 || t < N * TX) {
-            const int col = t % TX, e = t / TX;
-            if (col < ncol) {
-                C x = lds[e * TX + col];
-                if (nscale >= 1) x = scl(x, (RT)s1);
-                if (nscale >= 2) x = scl(x, (RT)s2);
-                if (nscale >= 3) x = scl(x, (RT)s3);
-                base[col + e * estride] = x;
-            }
-        }
-    }
+    auto get = [&](int e, int col) { return col < ncol ? base[col + e * estride] : mk<C>(RT(0), RT(0)); };
+    auto put = [&](int e, int col, C x) {
+        if (col >= ncol) return;
+        if (nscale >= 1) x = scl(x, (RT)s1);
+        if (nscale >= 2) x = scl(x, (RT)s2);
+        if (nscale >= 3) x = scl(x, (RT)s3);
+        base[col + e * estride] = x;
+    };
+    fft<N, TX, T, TX, 1, true, SIGN, PL, false, false>(lds, tw, get, put);
 }
 
 template <int N, int TX, int T, int SIGN, class C, int PL = 0>
@@ -740,41 +746,20 @@ __device__ __forceinline__ void zsolve_body(C *lds, int bx, int by, const C *__r
     const int64_t estride = (int64_t)nkxs * ny;
     C *base = data + kx0 + (int64_t)j * nkxs;
     const double *kb = ksqr + kx0 + (int64_t)j * nkx;
-#pragma unroll
-    for (int s = 0; s < (N * TX + T - 1) / T; ++s) {
-        const int t = (int)threadIdx.x + s * T;
-        if ((N * TX) % T == 0 || t < N * TX) {
-            const int col = t % TX, e = t / TX;
-            lds[e * TX + col] = (col < ncol) ? base[col + e * estride] : mk<C>(RT(0), RT(0));
-        }
-    }
-    __syncthreads();
-    fft<N, TX, T, TX, 1, true, -1, PL>(lds, tw);
-#pragma unroll
-    for (int s = 0; s < (N * TX + T - 1) / T; ++s) {
-        const int t = (int)threadIdx.x + s * T;
-        if ((N * TX) % T == 0 || t < N * TX) {
-            const int col = t % TX, e = t / TX;
-            if (col < ncol) {
-                const C xs = lds[e * TX + col];
-                double xr = (double)xs.x * dx * dy * dz, xi = (double)xs.y * dx * dy * dz;
-                const double ks = kb[col + e * (int64_t)nkx * ny];
-                if (ks > 0.0) { xr = -(xr / ks); xi = -(xi / ks); }
-                else { xr = 0.0; xi = 0.0; }
-                lds[e * TX + col] = mk<C>((RT)xr, (RT)xi);
-            }
-        }
-    }
-    __syncthreads();
-    fft<N, TX, T, TX, 1, true, +1, PL>(lds, tw);
-#pragma unroll
-    for (int s = 0; s < (N * TX + T - 1) / T; ++s) {
-        const int t = (int)threadIdx.x + s * T;
-        if ((N * TX) % T == 0 || t < N * TX) {
-            const int col = t % TX, e = t / TX;
-            if (col < ncol) base[col + e * estride] = lds[e * TX + col];
-        }
-    }
+    auto get = [&](int e, int col) { return col < ncol ? base[col + e * estride] : mk<C>(RT(0), RT(0)); };
+    auto solve = [&](int e, int col, C xs) {
+        double xr = (double)xs.x * dx * dy * dz, xi = (double)xs.y * dx * dy * dz;
+        const double ks = col < ncol ? kb[col + e * (int64_t)nkx * ny] : 0.0;
+        if (ks > 0.0) { xr = -(xr / ks); xi = -(xi / ks); }
+        else { xr = 0.0; xi = 0.0; }
+        lds[e * TX + col] = mk<C>((RT)xr, (RT)xi);
+    };
+    fft<N, TX, T, TX, 1, true, -1, PL, false, true>(lds, tw, get, solve);
+    fft<N, TX, T, TX, 1, true, +1, PL, true, false>(
+        lds, tw, [&](int e, int col) { return lds[e * TX + col]; },
+        [&](int e, int col, C x) {
+            if (col < ncol) base[col + e * estride] = x;
+        });
 }
 
 template <int N, int TX, int T, class C, int PL = 0>
@@ -797,9 +782,13 @@ constexpr int XROWS(int n2) { return n2 >= 1024 ? 1 : 1024 / n2; }
 template <class C> constexpr int TCOL = 64 / (int)sizeof(C);
 constexpr int TTHREADS = 256;
 template <class C> constexpr int TCOLS(int n) { return n * TCOL<C> / 16 > 256 ? n * TCOL<C> / 16 : 256; }
-// single-model passes: half the columns for the longest transforms (LDS per work-group)
-template <class C, int N> constexpr int TCOLN = N >= 1024 ? TCOL<C> / 2 : TCOL<C>;
-template <class C, int N> constexpr int TCOLSN = N * TCOLN<C, N> / 16 > 256 ? N * TCOLN<C, N> / 16 : 256;
+// single-model passes: four values per thread, one radix-4 butterfly, so that
+// a whole pass is in flight at once and short transforms leave no wavefront
+// idle; eight from 1024 on, whose work-groups of 512 threads share a CU better
+// than those of 1024 (1024x1024x64, y: 262 + 273 us; 269 + 285 with four; 341 +
+// 374 with half the columns, whose 32-byte segments each line is read in)
+constexpr int threads_of(int n) { return n <= 64 ? 64 : (n + 63) / 64 * 64; }
+template <class C, int N> constexpr int TCOLSN = threads_of(N * TCOL<C> / (N >= 1024 || N * TCOL<C> / 4 > 1024 ? 8 : 4));
 
 // plan 1 bodies are compiled for the FP32 transforms of lengths it changes
 template <int N, class RT> constexpr bool has_plan1 = std::is_same<RT, float>::value && plan_differs(N);
@@ -855,13 +844,13 @@ template <int N, class C, int PL>
 void launch_cols_pl(const C *tw, hipStream_t st, C *data, int nkx, int64_t estride, int64_t lstride,
                     unsigned ny_or_nz, int sign, double s1, double s2, double s3, int nscale)
 {
-    const dim3 grid((unsigned)((nkx + TCOLN<C, N> - 1) / TCOLN<C, N>), ny_or_nz);
+    const dim3 grid((unsigned)((nkx + TCOL<C> - 1) / TCOL<C>), ny_or_nz);
     constexpr int T = TCOLSN<C, N>;
     if (sign < 0)
-        hipLaunchKernelGGL((c2c_cols<N, TCOLN<C, N>, T, -1, C, PL>), grid, dim3(T), 0, st, tw, data, nkx, estride,
+        hipLaunchKernelGGL((c2c_cols<N, TCOL<C>, T, -1, C, PL>), grid, dim3(T), 0, st, tw, data, nkx, estride,
                            lstride, s1, s2, s3, nscale);
     else
-        hipLaunchKernelGGL((c2c_cols<N, TCOLN<C, N>, T, +1, C, PL>), grid, dim3(T), 0, st, tw, data, nkx, estride,
+        hipLaunchKernelGGL((c2c_cols<N, TCOL<C>, T, +1, C, PL>), grid, dim3(T), 0, st, tw, data, nkx, estride,
                            lstride, s1, s2, s3, nscale);
 }
 
@@ -881,15 +870,15 @@ bool launch_cols(const C *tw, hipStream_t st, C *data, int nkx, int64_t estride,
 template <int N, class C>
 bool launch_zsolve(Model &m, C *data, const C *tw, int nkxs, int plan)
 {
-    const dim3 grid((unsigned)((m.g.nkx + TCOLN<C, N> - 1) / TCOLN<C, N>), (unsigned)m.g.ny);
+    const dim3 grid((unsigned)((m.g.nkx + TCOL<C> - 1) / TCOL<C>), (unsigned)m.g.ny);
     constexpr int T = TCOLSN<C, N>;
     if constexpr (has_plan1<N, typename real_of<C>::type>)
         if (plan == 1) {
-            hipLaunchKernelGGL((z_periodic_solve<N, TCOLN<C, N>, T, C, 1>), grid, dim3(T), 0, m.stream, tw, data, m.ksqr,
+            hipLaunchKernelGGL((z_periodic_solve<N, TCOL<C>, T, C, 1>), grid, dim3(T), 0, m.stream, tw, data, m.ksqr,
                                m.g.nkx, nkxs, m.g.ny, m.prm.dx, m.prm.dy, m.prm.dz);
             return true;
         }
-    hipLaunchKernelGGL((z_periodic_solve<N, TCOLN<C, N>, T, C, 0>), grid, dim3(T), 0, m.stream, tw, data, m.ksqr,
+    hipLaunchKernelGGL((z_periodic_solve<N, TCOL<C>, T, C, 0>), grid, dim3(T), 0, m.stream, tw, data, m.ksqr,
                        m.g.nkx, nkxs, m.g.ny, m.prm.dx, m.prm.dy, m.prm.dz);
     return true;
 }
