@@ -309,10 +309,10 @@ void launch_ab_exchange(Model &m, int itt, int tau, int taum1, int taum2);
 // the wavemaker on the current buffers: q += dt*(cs*re + sn*im), interior
 void launch_wavemaker(Model &m, double cs, double sn);
 // background-flow advection and body force into the tendency slot tau (both
-// forms; mixed_fields: the FP32 hi fields to advect, default the canonical ones)
-void launch_background(Model &m, int tau, float *const *mixed_fields = nullptr);
-// mixed step with background forcing: friction, forcing on the post-friction
-// state, then Adams-Bashforth (the fused kernel's terms in three passes)
+// forms)
+void launch_background(Model &m, int tau);
+// mixed step with background forcing: friction, then forcing on the
+// post-friction state and Adams-Bashforth
 void launch_friction_forcing_ab_mixed(Model &m, int itt, int tau, int taum1, int taum2, double qc1, const float *d1,
                                       double qc2, const float *d2);
 bool fused_friction_ok(const Model &m);

@@ -692,18 +692,22 @@ __global__ __launch_bounds__(BX * BY) void k_background(StepConsts c, BgArgs<T> 
     a.db[o] = (T)db;
 }
 
-// Adams-Bashforth of the mixed form after a separate friction pass (models
-// with background forcing, whose terms need the post-friction state): from
-// the post-friction (hi, lo) pair P, x = P + (AB increment - dt grad(Q)) in
-// FP64, split back into (hi, lo), with the halo images of hi.  The same
-// terms as the fused kernel's final stage (fric_body<float>).
+// The forcing and the Adams-Bashforth update of the mixed form in one pass,
+// after a friction pass of its own (models with background forcing, whose
+// terms need the post-friction state): the forced tendency into slot tau, and
+// from the post-friction (hi, lo) pair P, x = P + (AB increment - dt grad(Q))
+// in FP64, split back into (hi, lo), with the halo images of hi.  The slot's
+// FP32 values and the terms of the fused kernel's final stage
+// (fric_body<float>).
+//
+// Bound: memory.  512x128x128: a pass for the forcing and one for the update
+// took 163 + 234 us, the two in one 370 us: the slot and the post-friction
+// fields are read once.
 struct AbMixedArgs {
     const float *ph[4], *pl[4];          // post-friction state
     float *oh[4], *ol[4];                // new state
-    const float *t0[4], *t1[4], *t2[4];  // slots tau, taum1, taum2
+    const float *t1[4], *t2[4];          // slots taum1, taum2
     double scale[4];
-    int64_t gstride[4];
-    double grd[4];
     double ca, cb, cc;
     int order;
     const float *d1, *d2;
@@ -711,33 +715,57 @@ struct AbMixedArgs {
     int halo;
 };
 
-__global__ __launch_bounds__(BX * BY) void k_ab_mixed(StepConsts c, AbMixedArgs a)
+__device__ __forceinline__ void background_ab_point_f(const StepConsts &c, const BgArgs<float> &bg,
+                                                      const AbMixedArgs &a, int i, int j, int k)
+{
+    const int64_t o = idx(c, i, j, k);
+    // every value is read before the first is written, see project_f_point
+    double p0[4];
+    float t1[4] = {}, t2[4] = {}, q1[4] = {}, q2[4] = {};   // q: the increments at the point, east, north, above
+    const int64_t qs[4] = {0, 1, c.X, c.XY};
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        p0[f] = (double)a.ph[f][o] + (double)a.pl[f][o];
+        if (a.order >= 2) t1[f] = a.t1[f][o];
+        if (a.order >= 3) t2[f] = a.t2[f][o];
+        if (a.d1) q1[f] = a.d1[o + qs[f]];
+        if (a.d1 && a.d2) q2[f] = a.d2[o + qs[f]];
+    }
+    double d[4];
+    bg_point<float>(c, bg, k, o, d[0], d[1], d[2], d[3]);
+    double q[4];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        q[f] = a.qc1 * (double)q1[f];
+        if (a.d2) q[f] += a.qc2 * (double)q2[f];
+    }
+    const double grd[3] = {c.rdx, c.rdy, c.rdz};
+    float *slot[4] = {bg.du, bg.dv, bg.dw, bg.db};
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        const float t0 = (float)d[f];
+        slot[f][o] = t0;
+        const double s = a.scale[f];
+        double ab;
+        if (a.order == 1) ab = s * (double)t0;
+        else if (a.order == 2) ab = s * (a.ca * (double)t0 - a.cb * (double)t1[f]);
+        else ab = s * (a.ca * (double)t0 + a.cb * (double)t1[f] + a.cc * (double)t2[f]);
+        double gq = 0.0;
+        if (f < 3 && a.d1) gq = s * ((q[f + 1] - q[0]) * grd[f]);
+        const double x = p0[f] + (ab - gq);
+        const float hi = (float)x;
+        a.oh[f][o] = hi;
+        a.ol[f][o] = (float)(x - (double)hi);
+        if (a.halo) write_images<float>(c, a.oh[f], i, j, k, hi, 0);
+    }
+}
+
+__global__ __launch_bounds__(BX * BY) void k_background_ab_f(StepConsts c, BgArgs<float> bg, AbMixedArgs a)
 {
     const int i = blockIdx.x * (int)blockDim.x + threadIdx.x + 1;
     const int j = blockIdx.y * (int)blockDim.y + threadIdx.y + 1;
     if (i > c.nx || j > c.ny) return;
-    const int k = (int)blockIdx.z % c.nz + 1, f = (int)blockIdx.z / c.nz;
-    const int64_t o = idx(c, i, j, k);
-    const double s = a.scale[f];
-    double ab;
-    if (a.order == 1) ab = s * (double)a.t0[f][o];
-    else if (a.order == 2) ab = s * (a.ca * (double)a.t0[f][o] - a.cb * (double)a.t1[f][o]);
-    else ab = s * (a.ca * (double)a.t0[f][o] + a.cb * (double)a.t1[f][o] + a.cc * (double)a.t2[f][o]);
-    double gq = 0.0;
-    const int64_t gs = a.gstride[f];
-    if (gs && a.d1) {
-        double qo = a.qc1 * (double)a.d1[o], qn = a.qc1 * (double)a.d1[o + gs];
-        if (a.d2) {
-            qo += a.qc2 * (double)a.d2[o];
-            qn += a.qc2 * (double)a.d2[o + gs];
-        }
-        gq = s * ((qn - qo) * a.grd[f]);
-    }
-    const double x = ((double)a.ph[f][o] + (double)a.pl[f][o]) + (ab - gq);
-    const float hi = (float)x;
-    a.oh[f][o] = hi;
-    a.ol[f][o] = (float)(x - (double)hi);
-    if (a.halo) write_images<float>(c, a.oh[f], i, j, k, hi, 0);
+    background_ab_point_f(c, bg, a, i, j, (int)blockIdx.z + 1);
 }
 
 __global__ __launch_bounds__(BX * BY) void k_ab(StepConsts c, AbArgs a)
@@ -863,6 +891,14 @@ __device__ __forceinline__ void background_ab_point(const StepConsts &c, const B
                                                     int i, int j, int k)
 {
     const int64_t o = idx(c, i, j, k);
+    // every value is read before the first is written, see project_f_point
+    double s0[4], t1[4] = {}, t2[4] = {};
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        s0[f] = a.src[f][o];
+        if (a.order >= 2) t1[f] = a.t1[f][o];
+        if (a.order >= 3) t2[f] = a.t2[f][o];
+    }
     double d[4];
     bg_point<double>(c, bg, k, o, d[0], d[1], d[2], d[3]);
     bg.du[o] = d[0];
@@ -874,11 +910,11 @@ __device__ __forceinline__ void background_ab_point(const StepConsts &c, const B
         const double s = a.scale[f];
         double val;
         if (a.order == 1) {
-            val = a.src[f][o] + s * d[f];
+            val = s0[f] + s * d[f];
         } else if (a.order == 2) {
-            val = a.src[f][o] + s * (a.ca * d[f] - a.cb * a.t1[f][o]);
+            val = s0[f] + s * (a.ca * d[f] - a.cb * t1[f]);
         } else {
-            val = a.src[f][o] + s * (a.ca * d[f] + a.cb * a.t1[f][o] + a.cc * a.t2[f][o]);
+            val = s0[f] + s * (a.ca * d[f] + a.cb * t1[f] + a.cc * t2[f]);
         }
         a.dst[f][o] = val;
         if (a.halo) write_images<double>(c, a.dst[f], i, j, k, val, 0);
@@ -1357,6 +1393,10 @@ __device__ __forceinline__ void project_f_point(const StepConsts &c, float *__re
     const double pe = dp[idx(c, i == c.nx ? 1 : i + 1, j, k)];
     const double pn = dp[idx(c, i, j == c.ny ? 1 : j + 1, k)];
     const double pt = dp[idx(c, i, j, k == c.nz ? (c.lid ? c.nz : 1) : k + 1)];
+    // every value is read before the first is written: behind a write that the
+    // compiler cannot tell from it, a read would wait for its turn
+    const double u0 = (double)uh[o] + (double)ul[o], v0 = (double)vh[o] + (double)vl[o];
+    const double w0 = (double)wh[o] + (double)wl[o], p0 = pint[o];
     // with halo set, the halo images of the hi parts, of the increment and of
     // pint are written too (Neumann in z under a lid for the last two)
     auto put = [&](float *h, float *l, double x) {
@@ -1365,11 +1405,10 @@ __device__ __forceinline__ void project_f_point(const StepConsts &c, float *__re
         l[o] = (float)(x - (double)hi);
         if (halo) write_images<float>(c, h, i, j, k, hi, 0);
     };
-    put(uh, ul, ((double)uh[o] + (double)ul[o]) - c.dt * ((pe - pc) * c.rdx));
-    put(vh, vl, ((double)vh[o] + (double)vl[o]) - c.dt * ((pn - pc) * c.rdy));
-    if (c.lid && k >= c.nz) put(wh, wl, 0.0);
-    else put(wh, wl, ((double)wh[o] + (double)wl[o]) - (c.dt / c.dsqr) * ((pt - pc) * c.rdz));
-    const double pn1 = pint[o] + pc;
+    put(uh, ul, u0 - c.dt * ((pe - pc) * c.rdx));
+    put(vh, vl, v0 - c.dt * ((pn - pc) * c.rdy));
+    put(wh, wl, (c.lid && k >= c.nz) ? 0.0 : w0 - (c.dt / c.dsqr) * ((pt - pc) * c.rdz));
+    const double pn1 = p0 + pc;
     pint[o] = pn1;
     if (halo) {
         write_images<float>(c, dp, i, j, k, (float)pc, c.lid);
@@ -1389,9 +1428,8 @@ __global__ __launch_bounds__(256) void k_project_f(StepConsts c, float *__restri
     const int r = xcd_remap((int)blockIdx.x + gx * ((int)blockIdx.y + gy * (int)blockIdx.z), gx * gy * (int)gridDim.z);
     const int i = (r % gx) * (int)blockDim.x + threadIdx.x + 1;
     const int j = ((r / gx) % gy) * (int)blockDim.y + threadIdx.y + 1;
-    const int k = r / (gx * gy) + 1;
     if (i > c.nx || j > c.ny) return;
-    project_f_point(c, uh, ul, vh, vl, wh, wl, dp, pint, i, j, k, halo);
+    project_f_point(c, uh, ul, vh, vl, wh, wl, dp, pint, i, j, r / (gx * gy) + 1, halo);
 }
 
 // host-layout conversions of the mixed form: 0 split FP64 -> (hi, lo),
@@ -1612,11 +1650,10 @@ __global__ __launch_bounds__(BX * BY) void k_ens_background_f(const EnsMember *_
 }
 
 // mixed forced members, the steady step: the forcing on the post-friction
-// hi parts of the third buffers into the FP32 slot tau (k_background<float>),
+// hi parts of the third buffers into the FP32 slot tau,
 // then the Adams-Bashforth update with the pressure-history term from the
 // third (hi, lo) buffers into the state's next buffers, halo images of the
-// hi parts included (k_ab_mixed) -- per point, with the slot's FP32 values,
-// so the same bits as the two kernels of a single model
+// hi parts included: k_background_ab_f of a single model
 __global__ __launch_bounds__(BX * BY) void k_ens_background_ab_f(const EnsMember *__restrict__ mem, EnsMap map,
                                                                   const EnsState *__restrict__ st)
 {
@@ -1639,61 +1676,37 @@ __global__ __launch_bounds__(BX * BY) void k_ens_background_ab_f(const EnsMember
     bg.ub = e.ub;
     bg.bb = e.bb;
     for (int q = 0; q < 4; ++q) bg.f[q] = e.bf[q];
-    const int64_t o = idx(c, i, j, k);
-    double fd[4];
-    bg_point<float>(c, bg, k, o, fd[0], fd[1], fd[2], fd[3]);
-    float sl[4];
-    for (int q = 0; q < 4; ++q) sl[q] = (float)fd[q];
-    bg.du[o] = sl[0];
-    bg.dv[o] = sl[1];
-    bg.dw[o] = sl[2];
-    bg.db[o] = sl[3];
     // the AB order and pressure-history coefficients of the step
     // (integrate_mixed of a single model)
-    int order;
-    double ca = 0.0, cb = 0.0, cc = 0.0, qc1 = 0.0, qc2 = 0.0;
+    AbMixedArgs a{};
     if (itt == 0) {
-        order = 1;
+        a.order = 1;
     } else if (itt == 1 || !e.ab3) {
-        order = 2;
-        ca = 1.5 + e.eps_ab;
-        cb = 0.5 + e.eps_ab;
-        qc1 = -(0.5 + e.eps_ab);
+        a.order = 2;
+        a.ca = 1.5 + e.eps_ab;
+        a.cb = 0.5 + e.eps_ab;
+        a.qc1 = -(0.5 + e.eps_ab);
     } else {
-        order = 3;
-        ca = 23.0 / 12.0;
-        cb = -16.0 / 12.0;
-        cc = 5.0 / 12.0;
-        qc1 = -16.0 / 12.0 + 5.0 / 12.0;
-        qc2 = 5.0 / 12.0;
+        a.order = 3;
+        a.ca = 23.0 / 12.0;
+        a.cb = -16.0 / 12.0;
+        a.cc = 5.0 / 12.0;
+        a.qc1 = -16.0 / 12.0 + 5.0 / 12.0;
+        a.qc2 = 5.0 / 12.0;
     }
-    const float *d1 = qc1 != 0.0 ? e.dpr[cur] : nullptr;
-    const float *d2 = qc2 != 0.0 ? e.dpr[(cur + 2) % 3] : nullptr;
+    a.d1 = a.qc1 != 0.0 ? e.dpr[cur] : nullptr;
+    a.d2 = a.qc2 != 0.0 ? e.dpr[(cur + 2) % 3] : nullptr;
     for (int f = 0; f < 4; ++f) {
-        const double s = (f == 2) ? c.dt / c.dsqr : c.dt;
-        const float *t1 = e.tf[f] + (int64_t)(st->taum1 - 1) * H;
-        const float *t2 = e.tf[f] + (int64_t)(st->taum2 - 1) * H;
-        double ab;
-        if (order == 1) ab = s * (double)sl[f];
-        else if (order == 2) ab = s * (ca * (double)sl[f] - cb * (double)t1[o]);
-        else ab = s * (ca * (double)sl[f] + cb * (double)t1[o] + cc * (double)t2[o]);
-        double gq = 0.0;
-        const int64_t gs = f == 0 ? 1 : (f == 1 ? c.X : (f == 2 ? c.XY : 0));
-        if (gs && d1) {
-            const double grd = f == 0 ? c.rdx : (f == 1 ? c.rdy : c.rdz);
-            double qo = qc1 * (double)d1[o], qn = qc1 * (double)d1[o + gs];
-            if (d2) {
-                qo += qc2 * (double)d2[o];
-                qn += qc2 * (double)d2[o + gs];
-            }
-            gq = s * ((qn - qo) * grd);
-        }
-        const double x = ((double)e.tmph[f][o] + (double)e.tmpl[f][o]) + (ab - gq);
-        const float hi = (float)x;
-        e.fh[f][par ^ 1][o] = hi;
-        e.fl[f][par ^ 1][o] = (float)(x - (double)hi);
-        write_images<float>(c, e.fh[f][par ^ 1], i, j, k, hi, 0);
+        a.ph[f] = e.tmph[f];
+        a.pl[f] = e.tmpl[f];
+        a.oh[f] = e.fh[f][par ^ 1];
+        a.ol[f] = e.fl[f][par ^ 1];
+        a.t1[f] = e.tf[f] + (int64_t)(st->taum1 - 1) * H;
+        a.t2[f] = e.tf[f] + (int64_t)(st->taum2 - 1) * H;
+        a.scale[f] = (f == 2) ? c.dt / c.dsqr : c.dt;
     }
+    a.halo = 1;
+    background_ab_point_f(c, bg, a, i, j, k);
 }
 
 __global__ __launch_bounds__(BX * BY) void k_ens_project(const EnsMember *__restrict__ mem, EnsMap map,
@@ -1749,7 +1762,10 @@ __global__ __launch_bounds__(TTHR, TendPlane<float>::WAVES) void k_ens_tendency_
     tendency_body<float>(c, a, g - map.start[mi]);
 }
 
-__global__ __launch_bounds__(FTHREADS, FricPlane<float>::WAVES) void k_ens_fric_f(const EnsMember *__restrict__ mem, EnsMap map,
+// (built for three work-groups per CU: with the members' records it spills at
+// the four of k_fric_ab<float>, 285 instead of 230 us for the 12 members of
+// 64x64x32, 96x96x48 and 128x128x64)
+__global__ __launch_bounds__(FTHREADS, 6) void k_ens_fric_f(const EnsMember *__restrict__ mem, EnsMap map,
                                                           const EnsState *__restrict__ st, int cold)
 {
     const int g = xcd_remap((int)blockIdx.x, map.start[map.n]);
@@ -2075,7 +2091,7 @@ static BgArgs<float> bg_args_mixed(Model &m, int tau, float *const *fields)
     return a;
 }
 
-void launch_background(Model &m, int tau, float *const *mixed_fields)
+void launch_background(Model &m, int tau)
 {
     if (!m.mixed) {
         const PointShape sh = point_shape(m.g);
@@ -2084,7 +2100,7 @@ void launch_background(Model &m, int tau, float *const *mixed_fields)
     } else {
         const PointShape sh = point_shape(m.g);
         hipLaunchKernelGGL(k_background<float>, sh.grid, sh.block, 0, m.stream, m.c,
-                           bg_args_mixed(m, tau, mixed_fields ? mixed_fields : m.fh));
+                           bg_args_mixed(m, tau, m.fh));
     }
     PS3D_HIP_CHECK(hipGetLastError());
 }
@@ -2403,7 +2419,6 @@ void launch_friction_forcing_ab_mixed(Model &m, int itt, int tau, int taum1, int
     // lo parts and the AB pass use interior points only)
     friction_ab_impl<float>(m, m.fh, m.fl, m.ah, m.al, m.tf, -1, tau, taum1, taum2, 0.0, nullptr, 0.0, nullptr,
                             HALO_KEEP);
-    launch_background(m, tau, m.ah);
     AbMixedArgs a{};
     const ps3d_params &p = m.prm;
     for (int f = 0; f < 4; ++f) {
@@ -2411,12 +2426,9 @@ void launch_friction_forcing_ab_mixed(Model &m, int itt, int tau, int taum1, int
         a.pl[f] = m.al[f];
         a.oh[f] = m.fh[f];
         a.ol[f] = m.fl[f];
-        a.t0[f] = m.tf[f] + (int64_t)(tau - 1) * m.g.H;
         a.t1[f] = m.tf[f] + (int64_t)(taum1 - 1) * m.g.H;
         a.t2[f] = m.tf[f] + (int64_t)(taum2 - 1) * m.g.H;
         a.scale[f] = (f == 2) ? p.dt / p.dsqr : p.dt;
-        a.gstride[f] = f == 0 ? 1 : (f == 1 ? m.g.X : (f == 2 ? m.g.XY : 0));
-        a.grd[f] = f == 0 ? m.c.rdx : (f == 1 ? m.c.rdy : m.c.rdz);
     }
     if (itt == 0) {
         a.order = 1;
@@ -2435,8 +2447,9 @@ void launch_friction_forcing_ab_mixed(Model &m, int itt, int tau, int taum1, int
     a.qc1 = qc1;
     a.qc2 = qc2;
     a.halo = m.fuse_halo ? 1 : 0;
-    const PointShape sh = point_shape(m.g, 4);
-    hipLaunchKernelGGL(k_ab_mixed, sh.grid, sh.block, 0, m.stream, m.c, a);
+    const PointShape sh = point_shape(m.g);
+    ProfScope ps(m, "ab_update");
+    hipLaunchKernelGGL(k_background_ab_f, sh.grid, sh.block, 0, m.stream, m.c, bg_args_mixed(m, tau, m.ah), a);
     PS3D_HIP_CHECK(hipGetLastError());
     if (!m.fuse_halo) {
         HaloArgsT<float> h{};
@@ -2507,11 +2520,8 @@ void launch_project_exchange(Model &m)
 {
     {
         ProfScope ps(m, "project");
-        const bool rows = m.g.nx >= 256;
-        const dim3 grid = rows ? dim3((unsigned)((m.g.nx + 255) / 256), (unsigned)m.g.ny, (unsigned)m.g.nz)
-                               : interior_grid(m.g);
-        hipLaunchKernelGGL(k_project, grid, rows ? dim3(256, 1) : dim3(BX, BY), 0, m.stream, m.c, m.u, m.v, m.w, m.p,
-                           m.fuse_halo ? 1 : 0);
+        const PointShape sh = point_shape(m.g);
+        hipLaunchKernelGGL(k_project, sh.grid, sh.block, 0, m.stream, m.c, m.u, m.v, m.w, m.p, m.fuse_halo ? 1 : 0);
         PS3D_HIP_CHECK(hipGetLastError());
     }
     if (m.fuse_halo) return;
@@ -2528,11 +2538,9 @@ void launch_project_exchange_f(Model &m, float *dp)
     // the next steps' pressure-history term
     {
         ProfScope ps(m, "project");
-        const bool rows = m.g.nx >= 256;
-        const dim3 grid = rows ? dim3((unsigned)((m.g.nx + 255) / 256), (unsigned)m.g.ny, (unsigned)m.g.nz)
-                               : interior_grid(m.g);
-        hipLaunchKernelGGL(k_project_f, grid, rows ? dim3(256, 1) : dim3(BX, BY), 0, m.stream, m.c, m.fh[0], m.fl[0],
-                           m.fh[1], m.fl[1], m.fh[2], m.fl[2], dp, m.pint, m.fuse_halo ? 1 : 0);
+        const PointShape sh = point_shape(m.g);
+        hipLaunchKernelGGL(k_project_f, sh.grid, sh.block, 0, m.stream, m.c, m.fh[0], m.fl[0], m.fh[1], m.fl[1],
+                           m.fh[2], m.fl[2], dp, m.pint, m.fuse_halo ? 1 : 0);
         PS3D_HIP_CHECK(hipGetLastError());
     }
     if (m.fuse_halo) return;
