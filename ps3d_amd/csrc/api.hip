@@ -360,7 +360,7 @@ std::vector<uint64_t> graph_signature(const Model &m, const int32_t *st)
     uint64_t h = 1469598103934665603ull;
     h = fnv(h, &m.c, sizeof(m.c));
     h = fnv(h, &m.prm, sizeof(m.prm));
-    const int opts[] = {m.tend_kc, m.fric_kc, m.thomas_cpw, (int)m.thomas_reg,
+    const int opts[] = {m.tend_kc, m.fric_kc, m.thomas_cpw,
                         (int)m.fuse_halo, m.fft_plan[0], m.fft_plan[1], m.fft_plan[2],
                         (int)m.bg_on, (int)m.bg_b_on, (int)m.bf_on[0], (int)m.bf_on[1], (int)m.bf_on[2],
                         (int)m.bf_on[3]};

@@ -230,14 +230,10 @@ struct Model {
     bool fuse_halo = false;
     // launch shapes (results do not depend on them; set by ps3d_tune):
     // levels per work-group of the k-marching kernels (0: heuristic) and
-    // the form of the Thomas solve (launch_thomas, launch_thomas_f: 1 whole
-    // columns in registers; 2 the real and imaginary parts of a column on two
-    // lanes; 16, 32, 64 columns per wave on the fly; -16, -32, -64 the factor
+    // the form of the Thomas solve (launch_thomas, launch_thomas_f: 1, 2
+    // columns in registers; 16, 32, 64 columns per wave on the fly; -16, -32, -64 the factor
     // tables; 0: the heuristic)
     int tend_kc = 0, fric_kc = 0, thomas_cpw = 0;
-    // the heuristic's first choice: whole columns in registers where nz is
-    // one of the compiled-in column lengths (k_thomas_reg)
-    bool thomas_reg = true;
     // ps3d_run's captured steps: a hipGraph of six steps (the period of the
     // tau rotation, the buffer parity and the pressure-increment ring) and
     // the signature of the state it was captured from
@@ -492,21 +488,15 @@ void ens_zsolve(hipStream_t s, const EnsMember *mem, const EnsMap &map, int nmax
 void ens_c2r(hipStream_t s, const EnsMember *mem, const EnsMap &map, size_t lds);
 // Thomas stage: ens_thomas_cols() columns per work-group; nz_max: most levels
 // of a rigid-lid member (sizes the LDS of the on-the-fly form)
-// reg: the register form (k_ens_thomas_reg, 64 columns per work-group), for
-// ensembles whose rigid-lid members all have thomas_reg_ok levels; split
-// (when not reg): the real and imaginary parts on two lanes
-// (k_ens_thomas_split, 32 columns per work-group), where they all have
-// thomas_split_ok levels
-int ens_thomas_cols(bool reg, bool split);
-// nz levels have a compiled-in register Thomas solve, and the spectral array
-// (fs_bytes) is addressed with 32-bit offsets
-bool thomas_reg_ok(int nz, uint64_t fs_bytes);
-// the same for the form with the real and imaginary parts on two lanes
-// (k_thomas_split), which has taller compiled-in lengths
+// split: the register form (k_ens_thomas_split), for ensembles whose rigid-lid
+// members all have thomas_split_ok levels
+int ens_thomas_cols(bool split);
+// a register Thomas solve takes nz levels, and the spectral array (fs_bytes) is
+// addressed with 32-bit offsets
 bool thomas_split_ok(int nz, uint64_t fs_bytes);
 // a compiled-in FP32 transform length whose plan 1 differs from plan 0
 bool fft_plan_choice(int n);
-void ens_thomas(hipStream_t s, const EnsMember *mem, const EnsMap &map, int nz_max, bool reg, bool split);
+void ens_thomas(hipStream_t s, const EnsMember *mem, const EnsMap &map, int nz_max, bool split);
 // the same stages for members of the mixed form.  cold: the provisional
 // Euler step of the cold start (tendency without the reference pressure,
 // friction + Euler); which: the increment a solve writes and a projection
@@ -524,7 +514,7 @@ void ens_r2c_f(hipStream_t s, const EnsMember *mem, const EnsMap &map, const Ens
 void ens_cols_y_f(hipStream_t s, const EnsMember *mem, const EnsMap &map, int sign, int nmax, size_t lds);
 void ens_zsolve_f(hipStream_t s, const EnsMember *mem, const EnsMap &map, int nmax, size_t lds);
 void ens_c2r_f(hipStream_t s, const EnsMember *mem, const EnsMap &map, const EnsState *st, int which, size_t lds);
-void ens_thomas_f(hipStream_t s, const EnsMember *mem, const EnsMap &map, int nz_max, bool reg, bool split);
+void ens_thomas_f(hipStream_t s, const EnsMember *mem, const EnsMap &map, int nz_max, bool split);
 // block counts and LDS bytes of the batched FFT stages for one member
 int ens_r2c_blocks(const EnsMember &e);
 int ens_cols_blocks(const EnsMember &e, int n_len, int lines);

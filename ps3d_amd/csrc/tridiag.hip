@@ -240,124 +240,48 @@ __global__ __launch_bounds__(64) void k_thomas_fly(C *__restrict__ fs, const dou
     thomas_col_fly<C>(fs, ksqr, ncols, nz, fxa, dz2, dsqr, col, dpl, cpl, cpw);
 }
 
-// The sweeps with whole columns in registers, NZ levels known at compile
-// time: one lane per column, 64 columns per wave.  Each lane loads its
-// column's NZ values at once (all loads in flight before the first is used),
-// keeps d'(k) in registers and c'(k) in LDS (NZ x 64 doubles), and stores
-// the solution.  With one wave per work-group and little LDS, every wave of
-// the solve is resident at once, so the sequential sweeps of all columns
-// run concurrently.  The arithmetic is that of thomas_col_fly, operation for
-// operation: the same bits.  C = double2: the FP64 path; C = float2: the
-// mixed form (FP32 right-hand side and solution, FP64 elimination).
-// cpl: NZ x 64 doubles of LDS; columns col (this lane's) of ncols.
-template <int NZ, class C>
-__device__ __forceinline__ void thomas_reg_col(C *__restrict__ fs, const double *__restrict__ ksqr, int64_t ncols,
-                                               int64_t col, double fxa, double dz2, double dsqr, double *cpl)
-{
-    double *cpk = cpl + threadIdx.x;   // c'(level q) at cpk[64 q]
-    // 32-bit byte offsets from the array base (the launchers check that FS
-    // is below 4 GiB), so each access is one base register pair plus one
-    // offset register
-    char *base = reinterpret_cast<char *>(fs);
-    constexpr uint32_t E = sizeof(C);
-    const uint32_t o0 = (uint32_t)col * E, st = (uint32_t)ncols * E;
-    double2 d[NZ];
-#pragma unroll
-    for (int k = 0; k < NZ; ++k) d[k] = to_d2(*reinterpret_cast<const C *>(base + (o0 + (uint32_t)k * st)));
-    const double ks = ksqr[col];
-    if (ks > 0) {
-        const double b1 = -ks - fxa;
-        double cprev = fxa / b1;
-        cpk[0] = cprev;
-        double2 dp = make_double2(d[0].x / b1, d[0].y / b1);
-        d[0] = dp;
-#pragma unroll
-        for (int q = 1; q < NZ; ++q) {
-            const int k = q + 1;   // level, 1-based
-            const double bk = (k == NZ) ? -ks - fxa : -ks - 2 * fxa;
-            const double mm = bk - cprev * fxa;
-            const double r = 1.0 / mm;
-            const double ck = (k == NZ) ? 0.0 : fxa * r;
-            cpk[64 * q] = ck;
-            cprev = ck;
-            const double2 e = d[q];
-            dp = make_double2((e.x - dp.x * fxa) * r, (e.y - dp.y * fxa) * r);
-            d[q] = dp;
-        }
-        double2 x = dp;
-        // c'(k) is read back from LDS (not kept in registers across the
-        // sweep); one wave per work-group, so the barrier holds nobody up
-        __syncthreads();
-#pragma unroll
-        for (int q = NZ - 2; q >= 0; --q) {
-            const double2 e = d[q];
-            const double c = cpk[64 * q];
-            x = make_double2(e.x - c * x.x, e.y - c * x.y);
-            d[q] = x;
-        }
-    } else {
-        // zero mode, pressure_solver.f90:44-50, as in thomas_col_fly
-        double2 pm1 = make_double2(0.0, 0.0);
-        double2 pk = make_double2(d[0].x * dz2 * dsqr, d[0].y * dz2 * dsqr);
-        double2 bk = d[1];
-        d[0] = pm1;
-        d[1] = pk;
-#pragma unroll
-        for (int k = 2; k < NZ; ++k) {
-            const double2 nxt = d[k];
-            const double2 pn = make_double2(2 * pk.x - pm1.x + bk.x * dz2 * dsqr,
-                                            2 * pk.y - pm1.y + bk.y * dz2 * dsqr);
-            d[k] = pn;
-            pm1 = pk;
-            pk = pn;
-            bk = nxt;
-        }
-    }
-    // the store offsets are formed here, one after the other (the empty asm
-    // makes each one opaque), rather than computed with the loads' and held
-    // in registers through both sweeps
-    uint32_t off = o0;
-#pragma unroll
-    for (int k = 0; k < NZ; ++k) {
-        asm volatile("" : "+v"(off));
-        *reinterpret_cast<C *>(base + off) = from_d2<C>(d[k]);
-        off += st;
-    }
-}
-
-template <int NZ, class C>
-__global__ __launch_bounds__(64, 1) void k_thomas_reg(C *__restrict__ fs, const double *__restrict__ ksqr,
-                                                      int64_t ncols, double fxa, double dz2, double dsqr)
-{
-    __shared__ double cpl[NZ * 64];
-    const int64_t col = (int64_t)xcd_remap((int)blockIdx.x, (int)gridDim.x) * 64 + threadIdx.x;
-    if (col >= ncols) return;
-    thomas_reg_col<NZ, C>(fs, ksqr, ncols, col, fxa, dz2, dsqr, cpl);
-}
-
-// Taller columns in registers: the real and imaginary parts of a column on
-// two neighbouring lanes (32 columns per wave), so a lane keeps NZ values of
-// d' instead of 2 NZ and columns of 128 levels still fit its registers.  Both
-// lanes of a column run its c' recurrence (the same operations on the same
-// operands, so the same bits; the even lane writes c' to LDS) and each runs
-// the d' sweeps of its part with the operations thomas_reg_col applies to
-// that component: the same bits as every other form.  R = double: the FP64
-// path; R = float: the mixed form (FP32 right-hand side and solution, FP64
-// elimination).  cpl: NZ x 32 doubles of LDS.
+// The sweeps with columns in registers: the real and imaginary parts of a
+// column on two neighbouring lanes (32 columns per wave), so that columns of
+// 128 levels fit a lane's registers.  Each lane loads its column's values at
+// once (all loads in flight before the first is used) and keeps d'(k) in
+// registers; c'(k) go to LDS.  With one wave per work-group and little LDS,
+// every wave of the solve is resident at once, so the sequential sweeps of all
+// columns run concurrently.  Both lanes of a column run its c' recurrence (the
+// same operations on the same operands, so the same bits; the even lane writes
+// c' to LDS) and each runs the d' sweeps of its part with the operations that
+// thomas_col_fly applies to that component: the same bits as every other form.
+// R = double: the FP64 path; R = float: the mixed form (FP32 right-hand side
+// and solution, FP64 elimination).  cpl: NZ x 32 doubles of LDS.
+//
+// Bound: the chain of a column (a division per level) on small grids, memory
+// on large ones: 160x120x37, on the fly with d' in LDS 20.4 us, so 11.8;
+// 256x256x100, 62 and 52 us; 1024x512x60, 149 and 114 us.  Whole columns on a
+// lane were slower at every length (128x128x64, 15.5 and 13.5 us; 512x256x64,
+// 34.7 and 31.3), and so was reading the factor tables instead of dividing
+// (256x256x37, 21.1 and 18.5 us; 512x256x40, 37 and 21), but for 0.7 us on
+// grids of 100x100x20 and less.
+// nz: the number of levels, up to NZ (a constant where they are equal).
 template <int NZ, class R>
 __device__ __forceinline__ void thomas_split_col(R *__restrict__ fs, const double *__restrict__ ksqr, int64_t ncols,
-                                                 int64_t col, double fxa, double dz2, double dsqr, double *cpl)
+                                                 int nz, int64_t col, double fxa, double dz2, double dsqr, double *cpl)
 {
     const int part = threadIdx.x & 1;
     double *cpk = cpl + (threadIdx.x >> 1);   // c'(level q) at cpk[32 q]
     // component `part` of column col at level k is element 2 (k ncols + col)
-    // + part; 32-bit byte offsets as in thomas_reg_col
+    // + part; 32-bit byte offsets from the array's base (the launchers check
+    // that FS is below 4 GiB), so that each access is one base register pair
+    // plus one offset register
     char *base = reinterpret_cast<char *>(fs);
     constexpr uint32_t E = sizeof(R);
     const uint32_t o0 = ((uint32_t)col * 2 + (uint32_t)part) * E, st = (uint32_t)ncols * 2 * E;
+    // (levels past the last one re-read it: no branch, and no conversion
+    // before the last load has been issued)
+    R raw[NZ];
+#pragma unroll
+    for (int k = 0; k < NZ; ++k) raw[k] = *reinterpret_cast<const R *>(base + (o0 + (uint32_t)min(k, nz - 1) * st));
     double d[NZ];
 #pragma unroll
-    for (int k = 0; k < NZ; ++k) d[k] = (double)*reinterpret_cast<const R *>(base + (o0 + (uint32_t)k * st));
+    for (int k = 0; k < NZ; ++k) d[k] = (double)raw[k];
     const double ks = ksqr[col];
     const bool solve = ks > 0;
     double x = 0.0;
@@ -369,15 +293,17 @@ __device__ __forceinline__ void thomas_split_col(R *__restrict__ fs, const doubl
         d[0] = dp;
 #pragma unroll
         for (int q = 1; q < NZ; ++q) {
-            const int k = q + 1;   // level, 1-based
-            const double bk = (k == NZ) ? -ks - fxa : -ks - 2 * fxa;
-            const double mm = bk - cprev * fxa;
-            const double r = 1.0 / mm;
-            const double ck = (k == NZ) ? 0.0 : fxa * r;
-            if (part == 0) cpk[32 * q] = ck;
-            cprev = ck;
-            dp = (d[q] - dp * fxa) * r;
-            d[q] = dp;
+            if (q < nz) {
+                const int k = q + 1;   // level, 1-based
+                const double bk = (k == nz) ? -ks - fxa : -ks - 2 * fxa;
+                const double mm = bk - cprev * fxa;
+                const double r = 1.0 / mm;
+                const double ck = (k == nz) ? 0.0 : fxa * r;
+                if (part == 0) cpk[32 * q] = ck;
+                cprev = ck;
+                dp = (d[q] - dp * fxa) * r;
+                d[q] = dp;
+            }
         }
         x = dp;
     }
@@ -390,11 +316,13 @@ __device__ __forceinline__ void thomas_split_col(R *__restrict__ fs, const doubl
     if (solve) {
 #pragma unroll
         for (int q = NZ - 2; q >= 0; --q) {
-            x = d[q] - cpk[32 * q] * x;
-            d[q] = x;
+            if (q <= nz - 2) {
+                x = d[q] - cpk[32 * q] * x;
+                d[q] = x;
+            }
         }
     } else {
-        // zero mode, pressure_solver.f90:44-50, as in thomas_reg_col
+        // zero mode, pressure_solver.f90:44-50, as in thomas_col_fly
         double pm1 = 0.0;
         double pk = d[0] * dz2 * dsqr;
         double bk = d[1];
@@ -402,66 +330,51 @@ __device__ __forceinline__ void thomas_split_col(R *__restrict__ fs, const doubl
         d[1] = pk;
 #pragma unroll
         for (int k = 2; k < NZ; ++k) {
-            const double nxt = d[k];
-            const double pn = 2 * pk - pm1 + bk * dz2 * dsqr;
-            d[k] = pn;
-            pm1 = pk;
-            pk = pn;
-            bk = nxt;
+            if (k < nz) {
+                const double nxt = d[k];
+                const double pn = 2 * pk - pm1 + bk * dz2 * dsqr;
+                d[k] = pn;
+                pm1 = pk;
+                pk = pn;
+                bk = nxt;
+            }
         }
     }
+    // the store offsets are formed here, one after the other (the empty asm
+    // makes each one opaque), rather than computed with the loads' and held
+    // in registers through both sweeps
     uint32_t off = o0;
 #pragma unroll
     for (int k = 0; k < NZ; ++k) {
         asm volatile("" : "+v"(off));
-        *reinterpret_cast<R *>(base + off) = (R)d[k];
+        if (k < nz) *reinterpret_cast<R *>(base + off) = (R)d[k];
         off += st;
     }
 }
 
-template <int NZ, class R>
-__global__ __launch_bounds__(64, 1) void k_thomas_split(R *__restrict__ fs, const double *__restrict__ ksqr,
-                                                        int64_t ncols, double fxa, double dz2, double dsqr)
+// Wavefronts per SIMD that the registers of NZ levels leave room for.  Two of
+// 64 levels cost a few spills and leave no second round of wavefronts where
+// there are more than four per CU (1024x512x60: 114 us with one, 95 with two);
+// of 32 levels four spill (64x64x32: 7.1 us with three, 8.1 with four).
+constexpr int split_waves(int nz) { return nz <= 40 ? 3 : nz <= 64 ? 2 : 1; }
+
+template <int NZ, bool EXACT, class R>
+__global__ __launch_bounds__(64, split_waves(NZ)) void k_thomas_split(R *__restrict__ fs, const double *__restrict__ ksqr,
+                                                        int64_t ncols, int nz, double fxa, double dz2, double dsqr)
 {
     __shared__ double cpl[NZ * 32];
     const int64_t col = (int64_t)xcd_remap((int)blockIdx.x, (int)gridDim.x) * 32 + (threadIdx.x >> 1);
     if (col >= ncols) return;
-    thomas_split_col<NZ, R>(fs, ksqr, ncols, col, fxa, dz2, dsqr, cpl);
+    thomas_split_col<NZ, R>(fs, ksqr, ncols, EXACT ? NZ : nz, col, fxa, dz2, dsqr, cpl);
 }
 
-// the same for the rigid-lid members of a batched ensemble, 64 columns per
-// work-group; every member's nz is one of the compiled-in lengths
-// (thomas_reg_ok), selected at run time
-template <class C>
-__global__ __launch_bounds__(64, 1) void k_ens_thomas_reg(const EnsMember *__restrict__ mem, EnsMap map)
+// the same for the rigid-lid members of a batched ensemble, 32 columns per
+// work-group, where every member has at most NMAX levels (64 or 128: the
+// registers of the tallest body bound the occupancy of every member)
+template <class C, int NMAX>
+__global__ __launch_bounds__(64, split_waves(NMAX)) void k_ens_thomas_split(const EnsMember *__restrict__ mem, EnsMap map)
 {
-    __shared__ double cpl[64 * 64];
-    const int g = xcd_remap((int)blockIdx.x, map.start[map.n]);
-    const int mi = ens_find(map, g);
-    const EnsMember &e = mem[mi];
-    const int64_t ncols = (int64_t)e.nkx * e.c.ny;
-    const int64_t col = (int64_t)(g - map.start[mi]) * 64 + threadIdx.x;
-    if (col >= ncols) return;
-    C *fs;
-    if constexpr (std::is_same<C, float2>::value) fs = e.FSf;
-    else fs = e.FS;
-    const double fxa = e.fxa, dz2 = e.c.dz * e.c.dz, dsqr = e.c.dsqr;
-    switch (e.c.nz) {
-    case 16: thomas_reg_col<16, C>(fs, e.ksqr, ncols, col, fxa, dz2, dsqr, cpl); break;
-    case 32: thomas_reg_col<32, C>(fs, e.ksqr, ncols, col, fxa, dz2, dsqr, cpl); break;
-    case 48: thomas_reg_col<48, C>(fs, e.ksqr, ncols, col, fxa, dz2, dsqr, cpl); break;
-    case 64: thomas_reg_col<64, C>(fs, e.ksqr, ncols, col, fxa, dz2, dsqr, cpl); break;
-    default: break;
-    }
-}
-
-// the split form for the rigid-lid members of a batched ensemble, 32
-// columns per work-group, where every member's nz is one of its compiled-in
-// lengths (thomas_split_ok) and some is too tall for k_ens_thomas_reg
-template <class C>
-__global__ __launch_bounds__(64, 1) void k_ens_thomas_split(const EnsMember *__restrict__ mem, EnsMap map)
-{
-    __shared__ double cpl[128 * 32];
+    __shared__ double cpl[NMAX * 32];
     using R = typename std::conditional<std::is_same<C, float2>::value, float, double>::type;
     const int g = xcd_remap((int)blockIdx.x, map.start[map.n]);
     const int mi = ens_find(map, g);
@@ -473,15 +386,16 @@ __global__ __launch_bounds__(64, 1) void k_ens_thomas_split(const EnsMember *__r
     if constexpr (std::is_same<C, float2>::value) fs = reinterpret_cast<R *>(e.FSf);
     else fs = reinterpret_cast<R *>(e.FS);
     const double fxa = e.fxa, dz2 = e.c.dz * e.c.dz, dsqr = e.c.dsqr;
-    switch (e.c.nz) {
-    case 16: thomas_split_col<16, R>(fs, e.ksqr, ncols, col, fxa, dz2, dsqr, cpl); break;
-    case 32: thomas_split_col<32, R>(fs, e.ksqr, ncols, col, fxa, dz2, dsqr, cpl); break;
-    case 48: thomas_split_col<48, R>(fs, e.ksqr, ncols, col, fxa, dz2, dsqr, cpl); break;
-    case 64: thomas_split_col<64, R>(fs, e.ksqr, ncols, col, fxa, dz2, dsqr, cpl); break;
-    case 96: thomas_split_col<96, R>(fs, e.ksqr, ncols, col, fxa, dz2, dsqr, cpl); break;
-    case 128: thomas_split_col<128, R>(fs, e.ksqr, ncols, col, fxa, dz2, dsqr, cpl); break;
-    default: break;
+    const int nz = e.c.nz;
+#define BODY(NZ, n) thomas_split_col<NZ, R>(fs, e.ksqr, ncols, n, col, fxa, dz2, dsqr, cpl)
+    if (nz <= 24) BODY(24, nz);
+    else if (nz <= 40) BODY(40, nz);
+    else if (nz <= 64) BODY(64, nz);
+    else if constexpr (NMAX > 64) {
+        if (nz <= 96) BODY(96, nz);
+        else BODY(128, nz);
     }
+#undef BODY
 }
 
 // the Thomas stage of a batched ensemble (rigid-lid members), ENS_TC columns
@@ -635,18 +549,11 @@ static void allow_lds(K kernel, size_t bytes)
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
 }
 
-bool thomas_reg_ok(int nz, uint64_t fs_bytes)
-{
-    return (nz == 16 || nz == 32 || nz == 48 || nz == 64) && fs_bytes < (uint64_t(1) << 32);
-}
+// the register form: up to 128 levels, FS below 4 GiB
+bool thomas_split_ok(int nz, uint64_t fs_bytes) { return nz >= 2 && nz <= 128 && fs_bytes < (uint64_t(1) << 32); }
 
-bool thomas_split_ok(int nz, uint64_t fs_bytes)
-{
-    return (nz == 16 || nz == 32 || nz == 48 || nz == 64 || nz == 96 || nz == 128) &&
-           fs_bytes < (uint64_t(1) << 32);
-}
-
-// the split register form (k_thomas_split) over data of element type R
+// the register form (k_thomas_split) over data of element type R; lengths that
+// grids often have are compiled in
 template <class R>
 static void launch_thomas_split(Model &m, R *data)
 {
@@ -654,14 +561,21 @@ static void launch_thomas_split(Model &m, R *data)
     const double fxa = 1.0 / (m.prm.dz * m.prm.dz) / m.prm.dsqr;
     const double dz2 = m.prm.dz * m.prm.dz, dsqr = m.prm.dsqr;
     const dim3 grid((unsigned)((ncols + 31) / 32));
-    switch (m.g.nz) {
-#define CASE(n)                                                                                                 \
-    case n:                                                                                                     \
-        hipLaunchKernelGGL((k_thomas_split<n, R>), grid, dim3(64), 0, m.stream, data, m.ksqr, ncols, fxa, dz2, dsqr); \
-        break;
+    const int nz = m.g.nz;
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(64), 0, m.stream, data, m.ksqr, ncols, nz, fxa, dz2, dsqr);
+    };
+    switch (nz) {
+#define CASE(n) case n: go(k_thomas_split<n, true, R>); break;
         CASE(16) CASE(32) CASE(48) CASE(64) CASE(96) CASE(128)
 #undef CASE
-    default: throw Error(PS3D_ERR_ARG, "split Thomas form: no compiled-in column length " + std::to_string(m.g.nz));
+    default:
+        if (nz <= 12) go(k_thomas_split<12, false, R>);
+        else if (nz <= 24) go(k_thomas_split<24, false, R>);
+        else if (nz <= 40) go(k_thomas_split<40, false, R>);
+        else if (nz <= 64) go(k_thomas_split<64, false, R>);
+        else if (nz <= 96) go(k_thomas_split<96, false, R>);
+        else go(k_thomas_split<128, false, R>);
     }
     PS3D_HIP_CHECK(hipGetLastError());
 }
@@ -682,28 +596,11 @@ void launch_thomas(Model &m, double2 *data)
     const double fxa = 1.0 / (m.prm.dz * m.prm.dz) / m.prm.dsqr;
     const int form = m.thomas_cpw;
     const uint64_t fsb = (uint64_t)m.g.S * sizeof(double2);
-    const bool reg = thomas_reg_ok(m.g.nz, fsb) && (form == 1 || (form == 0 && m.thomas_reg));
-    // form 2, or untuned where the whole-column form has no length: the
-    // real and imaginary parts on two lanes
-    if (!reg && thomas_split_ok(m.g.nz, fsb) && (form == 2 || (form == 0 && m.thomas_reg))) {
+    // untuned, and forms 1 and 2 (plans that were saved with a form of whole
+    // columns on a lane hold 1): columns in registers
+    if (thomas_split_ok(m.g.nz, fsb) && form >= 0 && form <= 2) {
         ProfScope ps(m, "thomas");
         launch_thomas_split<double>(m, reinterpret_cast<double *>(data));
-        return;
-    }
-    if (reg) {
-        const dim3 grid((unsigned)((ncols + 63) / 64));
-        const double dz2 = m.prm.dz * m.prm.dz, dsqr = m.prm.dsqr;
-        ProfScope ps(m, "thomas");
-        switch (m.g.nz) {
-#define CASE(n)                                                                                             \
-    case n:                                                                                                 \
-        hipLaunchKernelGGL((k_thomas_reg<n, double2>), grid, dim3(64), 0, m.stream, data, m.ksqr, ncols, fxa, dz2, \
-                           dsqr);                                                                           \
-        break;
-            CASE(16) CASE(32) CASE(48) CASE(64)
-#undef CASE
-        }
-        PS3D_HIP_CHECK(hipGetLastError());
         return;
     }
     // form: 16, 32, 64 columns per wave on the fly (c' and d' in LDS);
@@ -756,29 +653,12 @@ void launch_thomas_f(Model &m, float2 *data)
     const double fxa = 1.0 / (m.prm.dz * m.prm.dz) / m.prm.dsqr;
     const unsigned nb = (unsigned)((ncols + 63) / 64);
     ProfScope ps(m, "thomas");
-    // forms as in launch_thomas: 1 whole columns in registers, 2 the parts
-    // on two lanes, 32 on the fly, -64 the factor tables; 0 (untuned): the
-    // first of these that applies
+    // forms as in launch_thomas: 1, 2 columns in registers, 32 on the fly, -64
+    // the factor tables; 0 (untuned): the first of these that applies
     const int form = m.thomas_cpw;
     const uint64_t fsb = (uint64_t)m.g.S * sizeof(float2);
-    const bool reg = thomas_reg_ok(m.g.nz, fsb) && (form == 1 || (form == 0 && m.thomas_reg));
-    if (!reg && thomas_split_ok(m.g.nz, fsb) && (form == 2 || (form == 0 && m.thomas_reg))) {
+    if (thomas_split_ok(m.g.nz, fsb) && form >= 0 && form <= 2) {
         launch_thomas_split<float>(m, reinterpret_cast<float *>(data));
-        return;
-    }
-    if (reg) {
-        const dim3 grid((unsigned)((ncols + 63) / 64));
-        const double dz2 = m.prm.dz * m.prm.dz, dsqr = m.prm.dsqr;
-        switch (m.g.nz) {
-#define CASE(n)                                                                                             \
-    case n:                                                                                                 \
-        hipLaunchKernelGGL((k_thomas_reg<n, float2>), grid, dim3(64), 0, m.stream, data, m.ksqr, ncols, fxa, dz2,  \
-                           dsqr);                                                                           \
-        break;
-            CASE(16) CASE(32) CASE(48) CASE(64)
-#undef CASE
-        }
-        PS3D_HIP_CHECK(hipGetLastError());
         return;
     }
     // on the fly with 32 columns per wave where its LDS keeps several
@@ -801,14 +681,15 @@ void launch_thomas_f(Model &m, float2 *data)
     PS3D_HIP_CHECK(hipGetLastError());
 }
 
-int ens_thomas_cols(bool reg, bool split) { return reg ? 64 : (split ? 32 : ENS_TC); }
+int ens_thomas_cols(bool split) { return split ? 32 : ENS_TC; }
 
-void ens_thomas_f(hipStream_t s, const EnsMember *mem, const EnsMap &map, int nz_max, bool reg, bool split)
+void ens_thomas_f(hipStream_t s, const EnsMember *mem, const EnsMap &map, int nz_max, bool split)
 {
     if (!map.start[map.n]) return;
-    if (reg || split) {
-        if (reg) hipLaunchKernelGGL(k_ens_thomas_reg<float2>, dim3((unsigned)map.start[map.n]), dim3(64), 0, s, mem, map);
-        else hipLaunchKernelGGL(k_ens_thomas_split<float2>, dim3((unsigned)map.start[map.n]), dim3(64), 0, s, mem, map);
+    if (split) {
+        const dim3 grid((unsigned)map.start[map.n]);
+        if (nz_max <= 64) hipLaunchKernelGGL((k_ens_thomas_split<float2, 64>), grid, dim3(64), 0, s, mem, map);
+        else hipLaunchKernelGGL((k_ens_thomas_split<float2, 128>), grid, dim3(64), 0, s, mem, map);
         PS3D_HIP_CHECK(hipGetLastError());
         return;
     }
@@ -819,12 +700,13 @@ void ens_thomas_f(hipStream_t s, const EnsMember *mem, const EnsMap &map, int nz
     PS3D_HIP_CHECK(hipGetLastError());
 }
 
-void ens_thomas(hipStream_t s, const EnsMember *mem, const EnsMap &map, int nz_max, bool reg, bool split)
+void ens_thomas(hipStream_t s, const EnsMember *mem, const EnsMap &map, int nz_max, bool split)
 {
     if (!map.start[map.n]) return;
-    if (reg || split) {
-        if (reg) hipLaunchKernelGGL(k_ens_thomas_reg<double2>, dim3((unsigned)map.start[map.n]), dim3(64), 0, s, mem, map);
-        else hipLaunchKernelGGL(k_ens_thomas_split<double2>, dim3((unsigned)map.start[map.n]), dim3(64), 0, s, mem, map);
+    if (split) {
+        const dim3 grid((unsigned)map.start[map.n]);
+        if (nz_max <= 64) hipLaunchKernelGGL((k_ens_thomas_split<double2, 64>), grid, dim3(64), 0, s, mem, map);
+        else hipLaunchKernelGGL((k_ens_thomas_split<double2, 128>), grid, dim3(64), 0, s, mem, map);
         PS3D_HIP_CHECK(hipGetLastError());
         return;
     }

@@ -225,10 +225,8 @@ void tune_model(Model &m, int next_tau, const char *cache_path, int reps)
         }
     }
     if (m.prm.enable_vertical_boundaries && !cache.count("thomas " + sh)) {
-        // forms (launch_thomas, launch_thomas_f): 1 whole columns in
-        // registers (k_thomas_reg) and 2 the real and imaginary parts on two
-        // lanes (k_thomas_split), where nz is one of their compiled-in
-        // lengths; FP64: 16, 32, 64 columns per wave on the fly, whose LDS
+        // forms (launch_thomas, launch_thomas_f): 2 columns in registers
+        // (k_thomas_split), up to 128 levels; FP64: 16, 32, 64 columns per wave on the fly, whose LDS
         // keeps several work-groups on a CU (64 KiB; wider groups, which a
         // back-to-back timing can prefer, measured slower in the step), and
         // -16, -32, -64 the factor tables; mixed: 32 columns on the fly, and
@@ -238,7 +236,6 @@ void tune_model(Model &m, int next_tau, const char *cache_path, int reps)
         const size_t esz = mx ? sizeof(float2) : sizeof(double2);
         const uint64_t fsb = esz * (uint64_t)m.g.S;
         std::vector<int> forms;
-        if (thomas_reg_ok(m.g.nz, fsb)) forms.push_back(1);
         if (thomas_split_ok(m.g.nz, fsb)) forms.push_back(2);
         if (mx) {
             if ((sizeof(double2) + sizeof(double)) * 32 * (size_t)m.g.nz <= 160 * 1024) forms.push_back(32);
