@@ -523,14 +523,15 @@ int ps3d_ensemble_create(int n, const ps3d_params *prms, void *stream, ps3d_ense
             }
             // untuned levels per work-group: those of a single model with the
             // tiles of all members, which march together
-            int ttiles = 0, ftiles = 0;
+            int ttiles = 0, ftiles = 0, nz_max = 0;
             for (const EnsMember &e : E->tab) {
                 ttiles += e.tend_tx * e.tend_ty;
                 ftiles += e.fric_tx * e.fric_ty;
+                nz_max = std::max(nz_max, e.c.nz);
             }
             for (EnsMember &e : E->tab) {
                 set_chunks(e.c.nz, tendency_levels(ttiles, e.c.nz), e.tend_kc, e.tend_nchunk);
-                set_chunks(e.c.nz, friction_levels(ftiles, e.c.nz, E->mixed), e.fric_kc, e.fric_nchunk);
+                set_chunks(e.c.nz, friction_levels(ftiles, e.c.nz, E->mixed, nz_max), e.fric_kc, e.fric_nchunk);
             }
             bool split = true;
             for (ps3d_model *m : E->mem)

@@ -339,7 +339,7 @@ void launch_thomas_f(Model &m, float2 *data);
 // levels per work-group of the k-marching kernels when not tuned: tiles
 // column tiles march together over nz levels
 int tendency_levels(int tiles, int nz);
-int friction_levels(int tiles, int nz, bool mixed);
+int friction_levels(int tiles, int nz, bool mixed, int nz_max);
 void launch_friction_ab_raw(Model &m, int itt, int tau, int taum1, int taum2);
 // forced FP64 step: the fused friction chain alone into the second buffers
 // (halos pre-friction), marked current for the forcing and launch_ab_exchange

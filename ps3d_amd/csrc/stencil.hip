@@ -1503,7 +1503,9 @@ __global__ __launch_bounds__(TTHR, TendPlane<double>::WAVES) void k_ens_tendency
     tendency_body<double>(c, a, g - map.start[mi]);
 }
 
-__global__ __launch_bounds__(FTHREADS, FricPlane<double>::WAVES) void k_ens_fric(const EnsMember *__restrict__ mem, EnsMap map,
+// (built for four work-groups per CU, at the price of four spilled registers:
+// 270 -> 264 us for the 12 members of 64x64x32, 96x96x48 and 128x128x64)
+__global__ __launch_bounds__(FTHREADS, 8) void k_ens_fric(const EnsMember *__restrict__ mem, EnsMap map,
                                                         const EnsState *__restrict__ st)
 {
     const int g = xcd_remap((int)blockIdx.x, map.start[map.n]);
@@ -1959,16 +1961,20 @@ int tendency_levels(int tiles, int nz)
 }
 
 // Levels per work-group of the friction kernel: at least 1024 work-groups
-// (four per CU), of 2 to 8 levels (mixed form: to 16).  Short chunks keep the
-// tiles that share apron rows within reach of one L2: FP64, 512x512x64, 590
-// us with 8 levels, 617 with 16, 650 with 32, 683 with 64; 256x256x64, 131
-// with 8 or 16, 155 with 32.  Below 2 levels the three planes that a chunk
-// reads before its first level cost more than the work-groups give (64x64x32:
-// 13.2 us with 2, 14.4 with 1 or 4).  Mixed, 256x256x64: 137 us with 16, 144
-// with 8.
-int friction_levels(int tiles, int nz, bool mixed)
+// (four per CU), of 2 to 16 levels; in FP64 of at most 8 where 16 make more
+// than two rounds of work-groups.  Many rounds of short chunks keep the tiles
+// that share apron rows within reach of one L2 (512x512x64, 590 us with 8
+// levels, 617 with 16, 650 with 32, 683 with 64; 512x128x128, 309 with 8, 322
+// with 16); in one or two rounds all tiles march together anyway and the three
+// planes that a chunk reads before its first level are what counts
+// (256x256x64, 144 us with 16, 158 with 8; 128x128x128, 82 and 86).  Below 2
+// levels they cost more than the work-groups give (64x64x32: 13.2 us with 2,
+// 14.4 with 1 or 4).  Mixed, 256x256x64: 137 us with 16, 144 with 8.  nz_max:
+// the most levels of an ensemble's members (12 of 64x64x32, 96x96x48 and
+// 128x128x64: 264 us with 8 levels for all, 290 with 16 for the first).
+int friction_levels(int tiles, int nz, bool mixed, int nz_max)
 {
-    const int most = mixed ? 16 : 8;
+    const int most = mixed || 4 * tiles * ((nz_max + 15) / 16) <= 2048 ? 16 : 8;
     const int nchunk = std::max((nz + most - 1) / most, (1024 + 4 * tiles - 1) / (4 * tiles));
     return std::max(std::min(nz, 2), (nz + nchunk - 1) / nchunk);
 }
@@ -2270,7 +2276,7 @@ static void friction_ab_impl(Model &m, const T *const *in, const T *const *in_lo
     a.tiles_x = (g.nx + FTX - 1) / FTX;
     a.tiles_y = (g.ny + FTY - 1) / FTY;
     const int tiles = a.tiles_x * a.tiles_y;
-    a.kc = m.fric_kc > 0 ? m.fric_kc : friction_levels(tiles, g.nz, std::is_same<T, float>::value);
+    a.kc = m.fric_kc > 0 ? m.fric_kc : friction_levels(tiles, g.nz, std::is_same<T, float>::value, g.nz);
     a.nchunk = (g.nz + a.kc - 1) / a.kc;
     a.nblocks = tiles * a.nchunk * nf;
     a.halo = halo < 0 ? (m.fuse_halo ? HALO_IMAGES : HALO_NONE) : halo;
