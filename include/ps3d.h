@@ -136,7 +136,7 @@ int ps3d_synchronize(ps3d_model *m);
    the same bits.  (It chose between forming the tendencies of an unforced
    FP64 step inside the friction + Adams-Bashforth kernel and in a kernel of
    their own.  The separate kernels, which since read their planes straight
-   into LDS, are faster at every size: 200 against 400 us at 256x256x64.) */
+   into LDS, are faster: 200 against 400 us at 256x256x64.) */
 int ps3d_set_fused_tendency(ps3d_model *m, int on);
 
 /* Radix plans of a mixed-form model's FP32 transforms along x, y and z
@@ -251,9 +251,8 @@ int ps3d_fft_backward(ps3d_fft *f, const char *op, const double *qs, double *qp)
 
 /* Times the candidate launch shapes of this model's step on the live model
    (levels per work-group of the tendency and friction + AB kernels; the
-   form of the Thomas solve: whole columns in registers, the real and
-   imaginary parts on two lanes, columns per wavefront on the fly or with
-   factor tables; in the mixed form also the radix plan of each FP32
+   form of the Thomas solve: columns in registers, columns per wavefront on
+   the fly or with factor tables; in the mixed form also the radix plan of each FP32
    transform axis) and keeps the fastest; the choice is cached per (stage,
    grid, boundary, precision) in cache_path (NULL or "": none).
    next_tau is the slot the next step writes (it is used as scratch).  The

@@ -1,6 +1,6 @@
 // tune.hip -- autotuner of one model's launch shapes: levels per work-group
 // of the two k-marching kernels (tendency; friction + Adams-Bashforth), the
-// form of the Thomas solve (whole columns in registers, or columns per
+// form of the Thomas solve (columns in registers, or columns per
 // wavefront of the LDS form) and, in the mixed form, the radix plan of each
 // FP32 transform axis.  Each candidate is timed with
 // HIP events on the live model; the launches timed do not change the model's
