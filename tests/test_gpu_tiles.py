@@ -122,3 +122,29 @@ def test_steps_with_vertical_friction_bitwise(ops):
         assert np.array_equal(gpu.f[n], orc.f[n]), n
     gpu.close()
     orc.close()
+
+
+@pytest.mark.parametrize("nz", [4, 12, 13, 24, 25, 41, 63, 65, 97, 127, 129])
+def test_column_solve_lengths(nz):
+    """The column solve at the edges of its compiled-in bounds (12, 24, 40, 64,
+    96, 128 levels, and past the last): FP64 bit for bit like the oracle, alone
+    and as a member of an ensemble, whose tallest member picks its kernel."""
+    from ps3d_amd import configs
+    from ps3d_amd.ensemble import Ensemble
+    print(f"columns of {nz} levels", flush=True)
+    prm, gpu, orc = _pair(configs.random_state(16, 10, nz, lid=True, Avbi=0.0, Kvbi=0.0))
+    small, fields = configs.random_state(16, 8, 5, seed=9, lid=True, Avbi=0.0, Kvbi=0.0)
+    ens = Ensemble([prm, small])
+    for n in fields:
+        ens.set(0, n, orc.f[n])
+        ens.set(1, n, fields[n])
+    gpu.run(3)
+    orc.run(3)
+    ens.run(3)
+    gpu.pull()
+    for n in ("u", "v", "w", "b", "p"):
+        assert np.array_equal(gpu.f[n], orc.f[n]), n
+        assert np.array_equal(ens.get(0, n), orc.f[n]), n
+    ens.close()
+    gpu.close()
+    orc.close()
