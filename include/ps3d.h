@@ -160,7 +160,7 @@ int ps3d_get_fft_plan(ps3d_model *m, int32_t plans[3]);
    (ps3d_get_field / ps3d_set_field: u, v, w, b and du..db at tau hold the
    post-friction state there): the host round trip.  A nonzero return stops
    the step with PS3D_ERR_ARG.  While a hook or the wavemaker is set the
-   step takes the unfused friction kernels.  FP64 form only; fn = NULL
+   friction runs apart from the Adams-Bashforth update.  FP64 form only; fn = NULL
    removes the hook.  Replaces the config's set_forcing
    (the for_config files, e.g. lee_wave1.f90:232-331) for GPU runs. */
 typedef int (*ps3d_forcing_fn)(ps3d_model *m, void *user, int itt, int tau, void *stream);
