@@ -254,7 +254,7 @@ void enqueue_step_mixed(ps3d_ensemble &E, bool refine)
     ens_tendency_f(s, E.dev_tab, E.maps[S_TEND], E.dev_state, 0);
     ens_friction_ab_f(s, E.dev_tab, E.maps[S_FRIC], E.dev_state, 0);   // writes the halo images too
     // forced members (their friction went to the third (hi, lo) buffers, with
-    // the pre-friction hi halos): forcing + Adams-Bashforth
+    // the hi halos that in-place friction leaves): forcing + Adams-Bashforth
     ens_background_ab_f(s, E.dev_tab, E.maps[S_BGAB], E.dev_state);
     enqueue_solve_f(E, 1);
     ens_project_f(s, E.dev_tab, E.maps[S_PROJ], E.dev_state, 1);
@@ -277,7 +277,7 @@ void enqueue_step(ps3d_ensemble &E)
     ens_tendency(s, E.dev_tab, E.maps[S_TEND], E.dev_state);
     ens_friction_ab(s, E.dev_tab, E.maps[S_FRIC], E.dev_state);   // writes the halo images too
     // forced members (their friction went to the third buffers, with the
-    // pre-friction halos): set_forcing (integrate.f90:82) and AB
+    // halos that in-place friction leaves): set_forcing (integrate.f90:82) and AB
     ens_background_ab(s, E.dev_tab, E.maps[S_BGAB], E.dev_state);
     ens_r2c(s, E.dev_tab, E.maps[S_R2C], E.dev_state, E.lds_x);
     ens_cols_y(s, E.dev_tab, E.maps[S_COLS], -1, E.ny_max, E.lds_y);

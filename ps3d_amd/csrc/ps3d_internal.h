@@ -342,7 +342,7 @@ int tendency_levels(int tiles, int nz);
 int friction_levels(int tiles, int nz, bool mixed, int nz_max);
 void launch_friction_ab_raw(Model &m, int itt, int tau, int taum1, int taum2);
 // forced FP64 step: the fused friction chain alone into the second buffers
-// (halos pre-friction), marked current for the forcing and launch_ab_exchange
+// (halos as the in-place friction leaves them), marked current for the forcing and launch_ab_exchange
 void launch_friction_fused_only(Model &m);
 // then the background flow / body force and the AB update in one pass
 void launch_background_ab(Model &m, int itt, int tau, int taum1, int taum2);
@@ -472,8 +472,8 @@ struct EnsState {
 void ens_tendency(hipStream_t s, const EnsMember *mem, const EnsMap &map, const EnsState *st);
 void ens_friction_ab(hipStream_t s, const EnsMember *mem, const EnsMap &map, const EnsState *st);
 void ens_project(hipStream_t s, const EnsMember *mem, const EnsMap &map, const EnsState *st);
-// forced FP64 members: pre-friction halos into the third buffers (4 fields x
-// halo points per member), then forcing + AB (interior points per member)
+// forced FP64 members: forcing + AB from the third buffers, which the friction
+// stage has filled, halos included
 void ens_background_ab(hipStream_t s, const EnsMember *mem, const EnsMap &map, const EnsState *st);
 // mixed form: the forcing on the pre-friction state into slot tau (the cold
 // start's provisional step), and forcing + Adams-Bashforth from the third

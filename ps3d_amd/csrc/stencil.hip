@@ -610,7 +610,8 @@ __global__ __launch_bounds__(BX * BY) void k_wavemaker(StepConsts c, WaveArgs a,
 // the tendency slot tau at interior points.  The fluxes are the reference's
 // flux_east/north/top values, formed per face where needed (the lid zeroes
 // flux_top at k <= 0 and k >= nz); u, v, w, b are the post-friction fields,
-// whose halos still hold the pre-friction values, as in the reference.
+// whose halos still hold the pre-friction values (and zero for w from level
+// nz up, where the harmonic pass has cleared it), as in the reference.
 // The divisions and their association follow the reference's statements:
 // du and db as -Ro*(dfe/dx + dfn/dy + dft/dz), dv as -(Ro*dfe)/dx, dw as
 // -(dsqr*Ro*dfe)/dx.  T = float: the mixed form's version on the FP32 hi
@@ -993,17 +994,17 @@ struct FricArgs {
     const float *d1, *d2;
     double qc1, qc2;
     // HALO_IMAGES: also write the new values' halo images (integrate.f90:106-111);
-    // HALO_KEEP: out's halo takes in's values (the out-of-place friction leaves
-    // the halo that the reference's in-place passes leave); HALO_KEEP_TOP: so
-    // too, but zero from level nz on for a field with zero_top, as k_harmonic
-    // leaves it.  The copies are work-groups of their own at the end of the
-    // grid (hblocks per field): done by the tiles, the edge tiles become the
-    // slow ones and every tile pays in registers (512x128x128: 278 us; with a
-    // launch of its own 233 and 18 us; so 249 us.  FP32 202 and 16; so 188).
+    // HALO_KEEP: out's halo takes in's values, and zero from level nz on for a
+    // field with zero_top (integrate.f90:63): the halo that the reference's
+    // in-place passes leave, which set_forcing sees.  The copies are
+    // work-groups of their own at the end of the grid (hblocks per field): done
+    // by the tiles, the edge tiles become the slow ones and every tile pays in
+    // registers (512x128x128: 278 us; with a launch of its own 233 and 18 us;
+    // so 249 us.  FP32 202 and 16; so 188).
     int halo, hblocks;
 };
 constexpr int HALO_PT = FRIC_HALO / FTHREADS;
-enum { HALO_NONE = 0, HALO_IMAGES = 1, HALO_KEEP = 2, HALO_KEEP_TOP = 3 };
+enum { HALO_NONE = 0, HALO_IMAGES = 1, HALO_KEEP = 2 };
 
 // T = double: the drop-in, bit-exact.  T = float: the mixed form -- stencils
 // in FP32, and the new state (hi + lo) + harmonic increment + biharmonic
@@ -1280,10 +1281,10 @@ __device__ __forceinline__ void halo_ijk(const StepConsts &c, int64_t t64, int &
     }
 }
 
-// HALO_KEEP, HALO_KEEP_TOP: block hb of the halo copies of one field (hi
-// part), HALO_PT points per thread
+// HALO_KEEP: block hb of the halo copies of one field (hi part), HALO_PT
+// points per thread
 template <class T>
-__device__ __forceinline__ void keep_halo(const StepConsts &c, int halo, const FricField<T> &F, int hb)
+__device__ __forceinline__ void keep_halo(const StepConsts &c, const FricField<T> &F, int hb)
 {
     const int64_t nhalo = c.XY * (c.nz + 4) - (int64_t)c.nx * c.ny * c.nz;
     const int64_t t0 = (int64_t)hb * (FTHREADS * HALO_PT) + threadIdx.x;
@@ -1296,7 +1297,7 @@ __device__ __forceinline__ void keep_halo(const StepConsts &c, int halo, const F
         halo_ijk(c, min(t, nhalo - 1), i, j, k);
         o[s] = t < nhalo ? idx(c, i, j, k) : -1;
         v[s] = F.in[idx(c, i, j, k)];
-        if (halo == HALO_KEEP_TOP && F.zero_top && k >= c.nz) v[s] = T(0);
+        if (F.zero_top && k >= c.nz) v[s] = T(0);
     }
 #pragma unroll
     for (int s = 0; s < HALO_PT; ++s)
@@ -1308,7 +1309,7 @@ __global__ __launch_bounds__(FTHREADS, FricPlane<T>::WAVES) void k_fric_ab(StepC
 {
     if ((int)blockIdx.x >= a.nblocks) {
         const int hb = (int)blockIdx.x - a.nblocks;
-        keep_halo<T>(c, a.halo, a.f[hb / a.hblocks], hb % a.hblocks);
+        keep_halo<T>(c, a.f[hb / a.hblocks], hb % a.hblocks);
         return;
     }
     const int bid = xcd_remap((int)blockIdx.x, a.nblocks);
@@ -1506,6 +1507,12 @@ __global__ __launch_bounds__(TTHR, TendPlane<double>::WAVES) void k_ens_tendency
     tendency_body<double>(c, a, g - map.start[mi]);
 }
 
+// the harmonic pass clears w from level nz on under a rigid lid (integrate.f90:63)
+__device__ __forceinline__ int ens_zero_top(const EnsMember &e, int f)
+{
+    return (f == 2 && e.harm[0] && e.c.lid) ? 1 : 0;
+}
+
 // (built for four work-groups per CU, at the price of four spilled registers:
 // 270 -> 264 us for the 12 members of 64x64x32, 96x96x48 and 128x128x64)
 __global__ __launch_bounds__(FTHREADS, 8) void k_ens_fric(const EnsMember *__restrict__ mem, EnsMap map,
@@ -1524,7 +1531,8 @@ __global__ __launch_bounds__(FTHREADS, 8) void k_ens_fric(const EnsMember *__res
         FricField<double> F{};
         F.in = e.f[f][par];
         F.out = e.tmp[f];
-        keep_halo<double>(c, HALO_KEEP, F, hb % per);
+        F.zero_top = ens_zero_top(e, f);
+        keep_halo<double>(c, F, hb % per);
         return;
     }
     FricArgs<double> a{};   // tiling and AB coefficients; the field record is built alone
@@ -1555,7 +1563,7 @@ __global__ __launch_bounds__(FTHREADS, 8) void k_ens_fric(const EnsMember *__res
     F.Vm = e.Vm[q];
     F.bih = e.bih[q];
     F.Hbi = e.Hbi[q];
-    F.zero_top = (f == 2 && F.harm && c.lid) ? 1 : 0;
+    F.zero_top = ens_zero_top(e, f);
     a.halo = 1;
     if (e.forced) {
         // set_forcing sees the post-friction state (integrate.f90:82): the
@@ -1787,7 +1795,8 @@ __global__ __launch_bounds__(FTHREADS, 6) void k_ens_fric_f(const EnsMember *__r
         FricField<float> F{};
         F.in = e.fh[f][par];
         F.out = e.tmph[f];
-        keep_halo<float>(c, HALO_KEEP, F, hb % per);
+        F.zero_top = ens_zero_top(e, f);
+        keep_halo<float>(c, F, hb % per);
         return;
     }
     FricArgs<float> a{};
@@ -1829,7 +1838,7 @@ __global__ __launch_bounds__(FTHREADS, 6) void k_ens_fric_f(const EnsMember *__r
     F.Vm = e.Vm[q];
     F.bih = e.bih[q];
     F.Hbi = e.Hbi[q];
-    F.zero_top = (f == 2 && F.harm && c.lid) ? 1 : 0;
+    F.zero_top = ens_zero_top(e, f);
     F.gstride = f == 0 ? 1 : (f == 1 ? c.X : (f == 2 ? c.XY : 0));
     F.grd = f == 0 ? c.rdx : (f == 1 ? c.rdy : c.rdz);
     a.halo = 1;
@@ -2319,7 +2328,7 @@ static void friction_tiled(Model &m)
     }
     if (!fields) return;
     friction_ab_impl<double>(m, in, nullptr, out, nullptr, tend, -1, 1, 2, 3, 0.0, nullptr, 0.0, nullptr,
-                             HALO_KEEP_TOP, fields);
+                             HALO_KEEP, fields);
     for (int f = 0; f < 4; ++f) m.cur[f] ^= fields >> f & 1;
 }
 
@@ -2418,15 +2427,15 @@ void launch_friction_ab_mixed(Model &m, int itt, int tau, int taum1, int taum2, 
 }
 
 // the mixed step with background forcing: friction alone into the second
-// buffers (whose halos keep the pre-friction values, as the reference's
-// in-place friction leaves them), the forcing on that post-friction state
+// buffers (whose halos are those that the reference's in-place friction
+// leaves), the forcing on that post-friction state
 // into the tau slot, then the Adams-Bashforth pass back into the canonical
 // buffers
 void launch_friction_forcing_ab_mixed(Model &m, int itt, int tau, int taum1, int taum2, double qc1, const float *d1,
                                       double qc2, const float *d2)
 {
-    // the hi halos take the pre-friction values, which the forcing reads (the
-    // lo parts and the AB pass use interior points only)
+    // the hi halos are those that the forcing sees (HALO_KEEP; the lo parts
+    // and the AB pass use interior points only)
     friction_ab_impl<float>(m, m.fh, m.fl, m.ah, m.al, m.tf, -1, tau, taum1, taum2, 0.0, nullptr, 0.0, nullptr,
                             HALO_KEEP);
     AbMixedArgs a{};
@@ -2468,11 +2477,9 @@ void launch_friction_forcing_ab_mixed(Model &m, int itt, int tau, int taum1, int
     }
 }
 
-// the fused kernel alone, into the second buffers (no swap, no halo): the
-// autotuner's timing launch
 // integrate.f90:59-78 for a forced FP64 step without vertical biharmonic
 // friction: the fused kernel's friction chain alone (no AB) into the second
-// buffers, whose halos take the pre-friction values; the forcing and
+// buffers, with the halos that the in-place friction leaves; the forcing and
 // the Adams-Bashforth pass (launch_ab_exchange) read the second buffers
 void launch_friction_fused_only(Model &m)
 {
@@ -2485,6 +2492,8 @@ void launch_friction_fused_only(Model &m)
     for (int f = 0; f < 4; ++f) m.cur[f] = 1;
 }
 
+// the fused kernel alone, into the second buffers (no swap): the autotuner's
+// timing launch
 void launch_friction_ab_raw(Model &m, int itt, int tau, int taum1, int taum2)
 {
     if (m.mixed) {
