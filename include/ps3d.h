@@ -250,11 +250,14 @@ int ps3d_fft_backward(ps3d_fft *f, const char *op, const double *qs, double *qp)
 /* ---- launch-shape autotuner ------------------------------------------ */
 
 /* Times the candidate launch shapes of this model's step on the live model
-   (levels per work-group of the tendency and friction + AB kernels; the
-   form of the Thomas solve: columns in registers, columns per wavefront on
-   the fly or with factor tables; in the mixed form also the radix plan of each FP32
-   transform axis) and keeps the fastest; the choice is cached per (stage,
-   grid, boundary, precision) in cache_path (NULL or "": none).
+   (levels per work-group of the tendency and friction + AB kernels, the
+   untuned number among them; the form of the Thomas solve: columns in
+   registers, columns per wavefront on the fly or with factor tables; in the
+   mixed form also the radix plan of each FP32 transform axis) and keeps the
+   fastest; the choice is cached per (stage, grid, boundary, precision) in
+   cache_path (NULL or "": none).  Choices that the file holds are taken from
+   it and not timed again: a file that another version of the library wrote
+   is best removed.
    next_tau is the slot the next step writes (it is used as scratch).  The
    model's state is unchanged and results do not depend on the shapes.  No
    counterpart in the reference (its loop shapes are fixed by the compiler). */
@@ -410,8 +413,8 @@ int ps3d_ensemble_get_fft_plan(ps3d_ensemble *e, int member, int32_t plans[3]);
 int ps3d_ensemble_run(ps3d_ensemble *e, int nsteps, int32_t *state, int use_graph);
 int ps3d_ensemble_synchronize(ps3d_ensemble *e);
 /* Autotuner: times the candidate tile shapes of the k-marching stages
-   (levels per work-group of tendency and friction + AB) per member shape on
-   the live ensemble, keeps the fastest, and caches the choice per
+   (levels per work-group of tendency and friction + AB, the untuned numbers
+   among them) per member shape on the live ensemble, keeps the fastest, and caches the choice per
    (stage, nx x ny x nz, boundary, precision) in cache_path (NULL: no file).
    Results do not depend on the tile shapes. */
 int ps3d_ensemble_tune(ps3d_ensemble *e, const char *cache_path, int reps);

@@ -192,6 +192,18 @@ void upload_table(ps3d_ensemble &E)
     }
 }
 
+// untuned levels per work-group of a member with nz levels: those of a single
+// model with the tiles of all members, which march together
+int untuned_levels(const ps3d_ensemble &E, int stage, int nz)
+{
+    int tiles = 0, nz_max = 0;
+    for (const EnsMember &e : E.tab) {
+        tiles += stage == S_TEND ? e.tend_tx * e.tend_ty : e.fric_tx * e.fric_ty;
+        nz_max = std::max(nz_max, e.c.nz);
+    }
+    return stage == S_TEND ? tendency_levels(tiles, nz) : friction_levels(tiles, nz, E.mixed, nz_max);
+}
+
 void apply_tiles(ps3d_ensemble &E, int stage, const std::string &key, int kc)
 {
     for (size_t i = 0; i < E.mem.size(); ++i) {
@@ -521,17 +533,9 @@ int ps3d_ensemble_create(int n, const ps3d_params *prms, void *stream, ps3d_ense
                 E->mem[i] = m;
                 fill_member(E->tab[i], *m);
             }
-            // untuned levels per work-group: those of a single model with the
-            // tiles of all members, which march together
-            int ttiles = 0, ftiles = 0, nz_max = 0;
-            for (const EnsMember &e : E->tab) {
-                ttiles += e.tend_tx * e.tend_ty;
-                ftiles += e.fric_tx * e.fric_ty;
-                nz_max = std::max(nz_max, e.c.nz);
-            }
             for (EnsMember &e : E->tab) {
-                set_chunks(e.c.nz, tendency_levels(ttiles, e.c.nz), e.tend_kc, e.tend_nchunk);
-                set_chunks(e.c.nz, friction_levels(ftiles, e.c.nz, E->mixed, nz_max), e.fric_kc, e.fric_nchunk);
+                set_chunks(e.c.nz, untuned_levels(*E, S_TEND, e.c.nz), e.tend_kc, e.tend_nchunk);
+                set_chunks(e.c.nz, untuned_levels(*E, S_FRIC, e.c.nz), e.fric_kc, e.fric_nchunk);
             }
             bool split = true;
             for (ps3d_model *m : E->mem)
@@ -717,10 +721,7 @@ int ps3d_ensemble_tune(ps3d_ensemble *e, const char *cache_path, int reps)
                     int nz = 0;
                     for (ps3d_model *m : e->mem)
                         if (shape_key(m->prm) == sh) nz = m->g.nz;
-                    // levels per work-group: powers of two up to nz, and nz
-                    std::vector<int> cand;
-                    for (int kc = 1; kc < nz; kc *= 2) cand.push_back(kc);
-                    cand.push_back(nz);
+                    const std::vector<int> cand = tune_levels(untuned_levels(*e, stage, nz), nz);
                     // three interleaved rounds, the median of each
                     // candidate's (as the single-model tuner)
                     constexpr int kRounds = 3;

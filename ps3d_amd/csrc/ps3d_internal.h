@@ -355,6 +355,9 @@ void launch_divide_ksqr(Model &m, double2 *data);
 void balance_release(Model &m);
 // the single-model autotuner (tune.hip)
 void tune_model(Model &m, int next_tau, const char *cache_path, int reps);
+// the numbers of levels per work-group that the tuners time over nz levels:
+// the untuned choice, powers of two and nz
+std::vector<int> tune_levels(int untuned, int nz);
 // tuning cache files of "stage shape value" lines: read (missing file: empty;
 // malformed line: error) and written atomically (temporary file, rename)
 std::map<std::string, int> tune_cache_read(const char *path);

@@ -137,6 +137,18 @@ void tune_cache_write(const char *path, const std::map<std::string, int> &cache)
     }
 }
 
+// The untuned number is any from 1 to 16.  Of powers of two from two on alone,
+// tuning lost it: 64x64x32 stepped in 42.0 us untuned (one level) and in 43.1
+// tuned (two); with it in 41.3 and 41.3.  96x96x48 (three): 79.0 and 75.9.
+std::vector<int> tune_levels(int untuned, int nz)
+{
+    std::vector<int> c{untuned, nz};
+    for (int kc = 1; kc < nz; kc *= 2) c.push_back(kc);
+    std::sort(c.begin(), c.end());
+    c.erase(std::unique(c.begin(), c.end()), c.end());
+    return c;
+}
+
 void tune_model(Model &m, int next_tau, const char *cache_path, int reps)
 {
     PS3D_REQUIRE(next_tau >= 1 && next_tau <= 3, "tune: next_tau must be 1..3");
@@ -145,9 +157,7 @@ void tune_model(Model &m, int next_tau, const char *cache_path, int reps)
     std::map<std::string, int> cache = tune_cache_read(cache_path);
     const std::string sh = shape_of(m);
     const int nz = m.g.nz;
-    std::vector<int> levels;
-    for (int kc = 2; kc < nz; kc *= 2) levels.push_back(kc);
-    levels.push_back(nz);
+    auto tiles = [&](int tx, int ty) { return ((m.g.nx + tx - 1) / tx) * ((m.g.ny + ty - 1) / ty); };
     const int t1 = next_tau % 3 + 1, t2 = t1 % 3 + 1;   // any two other slots
 
     // flush: scratch for time_it_cold (null: back-to-back timing)
@@ -182,13 +192,13 @@ void tune_model(Model &m, int next_tau, const char *cache_path, int reps)
         cache[key] = best;
     };
 
-    pick("tendency", levels, m.tend_kc, reps, nullptr, [&] {
+    pick("tendency", tune_levels(tendency_levels(tiles(TEND_TX, TEND_TY), nz), nz), m.tend_kc, reps, nullptr, [&] {
         if (m.mixed) launch_tendency_mixed(m, next_tau, m.pint);
         else launch_tendency(m, next_tau);
     });
-    if (m.mixed || (fused_friction_ok(m)))
-        pick("friction_ab", levels, m.fric_kc, reps, nullptr,
-             [&] { launch_friction_ab_raw(m, 3, next_tau, t1, t2); });
+    if (m.mixed || fused_friction_ok(m))
+        pick("friction_ab", tune_levels(friction_levels(tiles(FRIC_TX, FRIC_TY), nz, m.mixed, nz), nz), m.fric_kc, reps,
+             nullptr, [&] { launch_friction_ab_raw(m, 3, next_tau, t1, t2); });
     if (m.mixed) {
         // radix plans of the FP32 transforms, on scratch arrays: the forward
         // x pass reads the state and writes the scratch spectrum, the other
