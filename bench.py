@@ -60,8 +60,8 @@ def algorithmic_bytes(name: str, prm, order: int = 3) -> float:
         "biharmonic_v": 2 * e * N,
         "ab_update": 4 * (2 + order) * e * N,  # per field R u, q slots  W u
         "friction_ab": 4 * (2 + order) * e * N,  # friction chain fused into the AB pass: same I/O
-        # tendency + friction + AB: per field R f and the q-1 older slots,
-        # W slot tau and the new f -- the same count
+        # one launch for tendency + friction + AB (the library has none): per
+        # field R f and the q-1 older slots, W slot tau and the new f
         "tend_friction_ab": 4 * (2 + order) * e * N,
         "fft_x_r2c": 3 * e * N + 2 * e * S,    # R u,v,w (divergence)  W FS
         "fft_y_fwd": 4 * e * S,                # R + W complex FS

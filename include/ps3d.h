@@ -395,8 +395,8 @@ int ps3d_ensemble_get_field(ps3d_ensemble *e, int member, int field, double *hos
    set it on a single model (lee_wave1.f90:239-314, a steady body force):
    background-flow advection and body force formed on the device from the
    post-friction state (integrate.f90:82).  Forced members run the friction
-   chain into a third set of buffers, then a halo copy and one forcing +
-   Adams-Bashforth stage (each one launch over the forced members), and stay
+   chain into a third set of buffers (in the launch of every member's), then
+   one forcing + Adams-Bashforth stage (one launch over them), and stay
    bit-identical to a single model of their form with the same forcing (in
    the mixed form the third buffers hold (hi, lo) pairs, and the cold start
    forms the forcing on the pre-friction state, as a single mixed model

@@ -7,17 +7,20 @@
 // with kx fastest.  The scalings of my_fft_2D/3D (QS*dx*dy(*dz)) and of
 // my_ifft_2D/3D (QP/(Lx*Ly(*Lz))) are applied inside the kernels.
 //
-// Layout on the device: every 1-D transform of a pass is staged in LDS,
-// batched so that global loads and stores are coalesced along the unit-stride
-// axis.  x-pass: 1 row per transform, rows of one k-level side by side.
-// y- and z-passes: TX consecutive kx columns per work-group, so each global
-// access touches TX*16 contiguous bytes; the transposition needed to run the
-// y (or z) transform on those columns happens in LDS, which is what the
-// pencil transposes of P3DFFT become on one device.
+// Layout on the device: every 1-D transform runs in one work-group, batched so
+// that global loads and stores are coalesced along the unit-stride axis.
+// x-pass: 1 row per transform, rows of one k-level side by side.  y- and
+// z-passes: TX consecutive kx columns per work-group, so each global access
+// touches TX*16 contiguous bytes; the transposition needed to run the y (or z)
+// transform on those columns happens in LDS, which is what the pencil
+// transposes of P3DFFT become on one device.
 //
 // Each pass is a Stockham autosort step on one LDS buffer: a thread reads the
 // R inputs of its butterflies into registers, the work-group synchronises,
-// and the outputs are written back in natural order.
+// and the outputs are written back in natural order.  Of the compiled-in
+// lengths, the y and z transforms take the first pass's inputs straight from
+// global memory and give the last pass's outputs straight to it, and c2r gives
+// its outputs so; r2c and the other lengths stage both sides in LDS.
 #include "ps3d_internal.h"
 
 #include <cmath>
@@ -784,9 +787,10 @@ constexpr int TTHREADS = 256;
 template <class C> constexpr int TCOLS(int n) { return n * TCOL<C> / 16 > 256 ? n * TCOL<C> / 16 : 256; }
 // single-model passes: four values per thread, one radix-4 butterfly, so that
 // a whole pass is in flight at once and short transforms leave no wavefront
-// idle; eight from 1024 on, whose work-groups of 512 threads share a CU better
-// than those of 1024 (1024x1024x64, y: 262 + 273 us; 269 + 285 with four; 341 +
-// 374 with half the columns, whose 32-byte segments each line is read in)
+// idle; eight from 1024 on, where four would make FP64 work-groups of 1024
+// threads, which share a CU worse than those of 512 (1024x1024x64, y: 262 + 273
+// us; 269 + 285 with four; 341 + 374 with half the columns, whose 32-byte
+// segments each line is read in), and FP32 ones of 2048
 constexpr int threads_of(int n) { return n <= 64 ? 64 : (n + 63) / 64 * 64; }
 template <class C, int N> constexpr int TCOLSN = threads_of(N * TCOL<C> / (N >= 1024 || N * TCOL<C> / 4 > 1024 ? 8 : 4));
 

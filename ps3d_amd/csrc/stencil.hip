@@ -941,15 +941,17 @@ __global__ __launch_bounds__(BX * BY) void k_background_ab(StepConsts c, BgArgs<
 // biharmonic_h to f1 and the AB update, writing a second buffer (neighbouring
 // tiles still read f0).
 //
-// Bound: memory, once enough of a CU's wavefronts are ready to issue.  A
-// plane comes in by one 16-byte direct-to-LDS load per lane, two levels ahead
-// of its use, instead of two loads to registers and two LDS writes: a tenth
-// fewer vector instructions, and 62 instead of 72 vector registers, so that
-// four work-groups fit a CU.  FP64, 256x256x64: 152 -> 131 us, 765 MB of
-// traffic (671 compulsory) at 5.8 TB/s, the rate of a streaming copy;
-// 512x512x64 672 -> 590 us; 1024x1024x128 5.77 -> 5.01 ms.  Mixed,
-// 256x256x64: 144 -> 137 us (79 registers, three work-groups per CU; at 64
-// registers it spills and takes 190 us).
+// Bound: memory on large grids, with half of the cycles spent issuing vector
+// instructions.  A plane comes in by one 16-byte direct-to-LDS load per lane,
+// two levels ahead of its use, instead of two loads to registers and two LDS
+// writes: a tenth fewer vector instructions, and 58 instead of 72 vector
+// registers, so that four work-groups fit a CU.  FP64, 256x256x64: in the step
+// 160 -> 149 us (142 tuned), 765 MB of traffic (671 compulsory) at 5.1 TB/s;
+// launched back to back 152 -> 131-138 us.  512x512x64 672 -> 590 us;
+// 1024x1024x128 5.77 -> 4.97 ms, 4.8 TB/s.  Mixed, 256x256x64: 145 -> 141 us
+// (136 tuned; 64 registers, four work-groups per CU).  Without the AB update
+// (order 0) half as many bytes go with the same instructions, whose issue
+// takes two thirds of the cycles: 512x128x128, 537 MB in 238-250 us.
 // ---------------------------------------------------------------------------
 constexpr int FTX = FRIC_TX, FTY = FRIC_TY;
 constexpr int R1X = FTX + 4, R1Y = FTY + 4;
@@ -1006,9 +1008,6 @@ struct FricArgs {
 constexpr int HALO_PT = FRIC_HALO / FTHREADS;
 enum { HALO_NONE = 0, HALO_IMAGES = 1, HALO_KEEP = 2 };
 
-// T = double: the drop-in, bit-exact.  T = float: the mixed form -- stencils
-// in FP32, and the new state (hi + lo) + harmonic increment + biharmonic
-// increment + AB increment summed in FP64 and split back into (hi, lo).
 // field of work-group bid: blocks run over (tile, chunk, field); mixed form
 // (tile, field, chunk), as u, v and w of a chunk read the same pressure
 // increments (256x256x64: 144.6 -> 141.3 us; FP64 148.5 -> 151)
@@ -1019,6 +1018,9 @@ __device__ __forceinline__ int fric_field(const FricArgs<T> &a, int bid)
     return __builtin_amdgcn_readfirstlane(std::is_same<T, float>::value ? r % a.nf : r / a.nchunk);
 }
 
+// T = double: the drop-in, bit-exact.  T = float: the mixed form -- stencils
+// in FP32, and the new state (hi + lo) + harmonic increment + biharmonic
+// increment + AB increment summed in FP64 and split back into (hi, lo).
 template <class T>
 __device__ __forceinline__ void fric_body(const StepConsts &c, const FricArgs<T> &a, const FricField<T> &F, int bid)
 {
