@@ -131,7 +131,7 @@ __global__ __launch_bounds__(BX * BY) void k_tendency(StepConsts c, const double
 // through its lower faces, which level k - 1 formed as its upper ones from
 // the same operands, and w.
 //
-// Bound: memory, at large grids (256x256x64: 280 MB in 53 us, 5.3 TB/s).
+// Bound: memory, at large grids (256x256x64: 296 MB in 52 us, 5.6 TB/s).
 // Planes come straight into LDS, as in fric_body, and what a level needs of
 // the one below is not recomputed: FP64 61 -> 53 us at 256x256x64, 2.36 ->
 // 2.01 ms at 1024x1024x128; mixed 60 -> 52 us.  The mixed form is built for

@@ -255,7 +255,7 @@ __global__ __launch_bounds__(64) void k_thomas_fly(C *__restrict__ fs, const dou
 //
 // Bound: the chain of a column (a division per level) on small grids, memory
 // on large ones: 160x120x37, on the fly with d' in LDS 20.4 us, so 11.8;
-// 256x256x100, 62 and 52 us; 1024x512x60, 149 and 114 us.  Whole columns on a
+// 256x256x100, 62 and 52 us; 1024x512x60, 149 and 95 us.  Whole columns on a
 // lane were slower at every length (128x128x64, 15.5 and 13.5 us; 512x256x64,
 // 34.7 and 31.3), and so was reading the factor tables instead of dividing
 // (256x256x37, 21.1 and 18.5 us; 512x256x40, 37 and 21), but for 0.7 us on
